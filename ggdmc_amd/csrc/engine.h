@@ -17,8 +17,8 @@
  *
  * Log-likelihood sums are canonical: chunk j of a subject is its trials
  * [j * kChunk, (j + 1) * kChunk); a 64-lane wave sums a chunk with lane l
- * holding term(j*kChunk + l) + term(j*kChunk + 64 + l) and a fixed xor
- * butterfly; a chain's log-likelihood is the sequential sum of its chunk sums
+ * holding the terms of trials j*kChunk + l and j*kChunk + 64 + l (batched
+ * path: one log of their densities' product) and a fixed xor butterfly; a chain's log-likelihood is the sequential sum of its chunk sums
  * in chunk order. How chains and trials are split over workgroups therefore
  * never changes a result bit.
  */

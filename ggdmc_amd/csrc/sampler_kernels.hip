@@ -32,7 +32,7 @@
 
 namespace ggdmc {
 
-/* 2^(j/64) for exp2_neg, staged into LDS by every kernel that evaluates the
+/* 2^(j/64) for exp_half_square, staged into LDS by every kernel that evaluates the
  * batched-path likelihood (load_exp2_table before its first barrier). */
 __shared__ double g_exp2tab[64];
 
@@ -42,7 +42,6 @@ __device__ __forceinline__ void load_exp2_table(const Dev &d) {
 
 struct DevOps {
     static __device__ __forceinline__ double exp2_frac(int j) { return g_exp2tab[j]; }
-    static __device__ __forceinline__ float exp2(float x) { return __builtin_amdgcn_exp2f(x); }
     static __device__ __forceinline__ float log2(float x) { return __builtin_amdgcn_logf(x); }
     static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
     /* the library's own FP64 functions (fp64_math.h), no math-library code */
@@ -64,9 +63,40 @@ __device__ __forceinline__ double trial_term(const AccK *kc, int n_acc, int w, d
                               : naive_trial_term<DevOps>(kc, n_acc, w, rt);
 }
 
+/* x of another lane of the wave: a DPP move within a row of 16 lanes, or the
+ * other half / neighbouring row by the gfx950 lane swaps (the two results of a
+ * swap of x with itself hold, per lane, x of the lane's own and of its partner
+ * group; their sum does not depend on which is which). */
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double x) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)u, CTRL, 0xF, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), CTRL, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+template <int LANES>
+__device__ __forceinline__ double swap_sum(double x) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t l = (uint32_t)u, h = (uint32_t)(u >> 32);
+    const auto a = LANES == 32 ? __builtin_amdgcn_permlane32_swap(l, l, false, false)
+                               : __builtin_amdgcn_permlane16_swap(l, l, false, false);
+    const auto b = LANES == 32 ? __builtin_amdgcn_permlane32_swap(h, h, false, false)
+                               : __builtin_amdgcn_permlane16_swap(h, h, false, false);
+    return __builtin_bit_cast(double, ((uint64_t)b[0] << 32) | a[0]) +
+           __builtin_bit_cast(double, ((uint64_t)b[1] << 32) | a[1]);
+}
+
+/* Sum over the wave by the xor butterfly of strides 32, 16, 8, 4, 2, 1, in
+ * vector registers. After the step of stride 8 a row's values repeat with
+ * period 8, so a rotation by 4 pairs the same values as xor 4. */
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v = swap_sum<32>(v);
+    v = swap_sum<16>(v);
+    v += dpp_f64<0x128>(v);   /* row_ror:8 */
+    v += dpp_f64<0x124>(v);   /* row_ror:4 */
+    v += dpp_f64<0x4E>(v);    /* quad_perm [2,3,0,1] */
+    v += dpp_f64<0xB1>(v);    /* quad_perm [1,0,3,2] */
     return v;
 }
 
@@ -112,13 +142,14 @@ struct TrialView {
     int64_t origin;
 };
 
-/* The terms a lane adds to its chunk sum: trials i1 and i1 + 64 of the
- * chunk (zero past t_end). MODE_MIXED: ill1 / ill2 report trials whose mixed
- * evaluation is ill-conditioned, and fix: those trials are evaluated with the
- * reference formula instead (the fix-up pass). */
+/* A lane's share of its chunk sum: the terms of trials i1 and i1 + 64 of the
+ * chunk (zero past t_end). MODE_MIXED: one log of the product of the two
+ * densities (above 1e-244, see mixed_density); ill reports a trial whose mixed
+ * evaluation is ill-conditioned, and with FIX (the fix-up pass) such a trial's
+ * term is the reference formula's and the other's its own log. */
 template <int MODE, bool FIX>
-__device__ __forceinline__ void lane_terms(const Dev &d, const TrialView &tv, const AccK *kc, int64_t base, int64_t t_end,
-                                           double &a, double &b, bool &ill1, bool &ill2) {
+__device__ __forceinline__ double lane_terms(const Dev &d, const TrialView &tv, const AccK *kc, int64_t base,
+                                             int64_t t_end, bool &ill) {
     const int lane = threadIdx.x & 63;
     const int64_t i1 = base + lane, i2 = i1 + 64;
     const bool h1 = i1 < t_end, h2 = i2 < t_end;
@@ -129,23 +160,25 @@ __device__ __forceinline__ void lane_terms(const Dev &d, const TrialView &tv, co
     const int code1 = tv.code[r1], code2 = tv.code[r2];
     const double rt1 = tv.rt[r1], rt2 = tv.rt[r2];
     const AccK *k1 = kc + (code1 >> 3) * d.n_acc, *k2 = kc + (code2 >> 3) * d.n_acc;
-    a = b = 0.0;
-    ill1 = ill2 = false;
+    ill = false;
     if (MODE == MODE_MIXED) {
-        double ma, mb;
-        mixed_trial_term_flagged2<DevOps>(k1, code1 & 7, rt1, k2, code2 & 7, rt2, d.n_acc, ma, mb, ill1, ill2);
+        double d1, d2;
+        bool ill1 = false, ill2 = false;
+        mixed_density2<DevOps>(k1, code1 & 7, rt1, k2, code2 & 7, rt2, d.n_acc, d1, d2, ill1, ill2);
         ill1 = h1 && ill1;
         ill2 = h2 && ill2;
-        a = h1 ? ma : 0.0;
-        b = h2 ? mb : 0.0;
+        ill = ill1 || ill2;
+        double v = mixed_log<DevOps>((h1 && !ill1 ? d1 : 1.0) * (h2 && !ill2 ? d2 : 1.0));
         if constexpr (FIX) {
-            if (ill1) a = naive_trial_term<DevOps>(k1, d.n_acc, code1 & 7, rt1);
-            if (ill2) b = naive_trial_term<DevOps>(k2, d.n_acc, code2 & 7, rt2);
+            if (ill1) v += naive_trial_term<DevOps>(k1, d.n_acc, code1 & 7, rt1);
+            if (ill2) v += naive_trial_term<DevOps>(k2, d.n_acc, code2 & 7, rt2);
         }
-    } else {
-        if (h1) a = naive_trial_term<DevOps>(k1, d.n_acc, code1 & 7, rt1);
-        if (h2) b = naive_trial_term<DevOps>(k2, d.n_acc, code2 & 7, rt2);
+        return v;
     }
+    double a = 0.0, b = 0.0;
+    if (h1) a = naive_trial_term<DevOps>(k1, d.n_acc, code1 & 7, rt1);
+    if (h2) b = naive_trial_term<DevOps>(k2, d.n_acc, code2 & 7, rt2);
+    return a + b;
 }
 
 /* Canonical chunk sums (see engine.h): C[c * c_stride + jj] for chains c < kb
@@ -175,14 +208,12 @@ __device__ __forceinline__ void chunk_sums(const Dev &d, const TrialView &tv, in
         double v = 0.0;
         if (active[c]) {
             const AccK *kc = reinterpret_cast<const AccK *>(acck) + (size_t)c * per_chain;
-            double a, b;
-            bool ill1, ill2;
-            lane_terms<MODE, false>(d, tv, kc, t0 + (int64_t)(j_lo + jj) * kChunk, t_end, a, b, ill1, ill2);
-            if (MODE == MODE_MIXED && __builtin_expect(__builtin_amdgcn_ballot_w64(ill1 || ill2) != 0, 0)) {
+            bool ill;
+            v = lane_terms<MODE, false>(d, tv, kc, t0 + (int64_t)(j_lo + jj) * kChunk, t_end, ill);
+            if (MODE == MODE_MIXED && __builtin_expect(__builtin_amdgcn_ballot_w64(ill) != 0, 0)) {
                 if (lane == 0) atomicOr(pend + (u >> 5), 1u << (u & 31));
                 continue;
             }
-            v = a + b;
         }
         v = wave_sum(v);
         if (lane == 0) C[(size_t)c * c_stride + jj] = v;
@@ -193,10 +224,8 @@ __device__ __forceinline__ void chunk_sums(const Dev &d, const TrialView &tv, in
             if (__builtin_expect(((pend[u >> 5] >> (u & 31)) & 1u) == 0, 1)) continue;
             const int c = u / nj, jj = u - c * nj;
             const AccK *kc = reinterpret_cast<const AccK *>(acck) + (size_t)c * per_chain;
-            double a, b;
-            bool ill1, ill2;
-            lane_terms<MODE, true>(d, tv, kc, t0 + (int64_t)(j_lo + jj) * kChunk, t_end, a, b, ill1, ill2);
-            const double v = wave_sum(a + b);
+            bool ill;
+            const double v = wave_sum(lane_terms<MODE, true>(d, tv, kc, t0 + (int64_t)(j_lo + jj) * kChunk, t_end, ill));
             if (lane == 0) C[(size_t)c * c_stride + jj] = v;
         }
     }
