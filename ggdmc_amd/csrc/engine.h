@@ -143,6 +143,17 @@ struct SweepArgs {
                              order (items carry group 0); else one group per item */
 };
 
+/* Work split of a likelihood call: n vectors over nj chunks of ntrial trials,
+ * sp.k vectors x jper chunks per workgroup of `threads`, nsplit workgroups per
+ * k vectors. */
+constexpr int kLoglikeBlock = 512; /* most threads per workgroup */
+struct LoglikeSplit {
+    int32_t n, k, nj, jper, nsplit, threads;
+    int32_t cmax;    /* chunk sums per vector held in LDS at once */
+    int32_t tstage;  /* trials staged in LDS (0: read from HBM) */
+    int64_t ntrial;
+};
+
 } // namespace ggdmc
 
 #endif

@@ -54,8 +54,8 @@ hipError_t ggdmc_internal_launch_store(const Dev *d, uint32_t iter, int subjects
                                       hipStream_t stream);
 hipError_t ggdmc_internal_launch_hyper_stats(const Dev *d, const double *rows, int S, int f,
                                              hipStream_t stream);
-hipError_t ggdmc_internal_launch_loglike(const Dev *d, const double *thetas, int nq, int s,
-                                         int mode, int cmax, size_t lds, hipStream_t stream,
+hipError_t ggdmc_internal_launch_loglike(const Dev *d, const LoglikeSplit *sp, const double *thetas, int mode,
+                                         size_t lds, hipStream_t stream, double *csum, uint32_t *ctr,
                                          double *out);
 }
 
@@ -1352,6 +1352,55 @@ int ggdmc_loglike_noalloc(const ggdmc_model *model, const ggdmc_subject *data, c
 
 } // extern "C"
 
+/* The split of a likelihood call. Per workgroup the constants take about 4 us
+ * whatever k, a chunk of one vector about 3 us of one wave; about 3 workgroups
+ * of 4 waves are resident on a CU. Times of whole calls, about 50 us of each
+ * outside the kernel:
+ *   - few vectors and chunks (at most 8 chunks per CU): one workgroup of 8
+ *     waves per vector and 8 chunks, one chunk a wave, so that the call is one
+ *     set-up and one chunk long (1 x 768: 55.5 us, 4 waves in two rounds 60.6);
+ *   - two vectors per CU or more: 4 waves and whole vectors, k of them together
+ *     while a wave has less than 6 chunks and 3.5 workgroups per CU remain, for
+ *     one set-up per k (8190 x 768: k = 1 176 us, 2 159, 4 153; 2000 x 768: 84,
+ *     80, 82; 624 x 768: 65, 66, 69; 1000 x 2047 of 4 accumulators: 93, 99,
+ *     114);
+ *   - a long subject under few vectors: 4 waves and 16 chunks (4 a wave), fewer
+ *     while that leaves less than 3 workgroups per CU (33 x 100608 of 4
+ *     accumulators: 4 chunks 197 us, 8 to 24 181, 48 198, one workgroup per
+ *     vector 804; 4 x 100608: 4 and 8 chunks 132, 16 138, 32 150).
+ * The first stages its trials in LDS with the set-up's loads; the others read
+ * them from L2 as they go (staged: 1000 x 2047 93 us instead of 90).
+ * may_split false: no chunk sums in memory, whole vectors only. */
+static LoglikeSplit loglike_split(int n, int64_t ntrial, int per_chain, int P, bool may_split) {
+    LoglikeSplit sp{};
+    sp.n = n;
+    sp.ntrial = ntrial;
+    sp.nj = (int)((ntrial + kChunk - 1) / kChunk);
+    const int nj = std::max(sp.nj, 1);
+    const int64_t cus = std::max(device_cus(), 1);
+    sp.k = 1;
+    sp.threads = 256;
+    sp.jper = nj;
+    if (may_split && (int64_t)n * ((nj + 7) / 8) <= cus) {
+        sp.jper = std::min(nj, 8);
+        sp.threads = nj > 4 ? 512 : 256;
+        sp.tstage = (int)std::min<int64_t>((int64_t)sp.jper * kChunk, ntrial);
+    } else if (n >= 2 * cus || !may_split) {
+        while (sp.k < 4 && sp.k * nj < 24 && n / (sp.k + 1) >= 7 * cus / 2) ++sp.k;
+    } else {
+        sp.jper = std::min(nj, 16);
+        while (sp.jper > 4 && (int64_t)n * ((nj + sp.jper - 1) / sp.jper) < 3 * cus) sp.jper -= 4;
+    }
+    sp.nsplit = (nj + sp.jper - 1) / sp.jper;
+    sp.cmax = std::min(sp.jper, sp.nsplit > 1 ? 256 : 1024 / sp.k);
+    if (sp.nsplit > 1) sp.cmax = std::max(sp.cmax, std::min(nj, 256));
+    const size_t soft = 40 * 1024;
+    auto bytes = [&]() { return ggdmc_internal_sweep_lds(1, P, sp.k, per_chain, sp.k, sp.cmax, sp.tstage); };
+    while (sp.k > 1 && bytes() > soft) --sp.k;
+    if (bytes() > soft) sp.tstage = 0;
+    return sp;
+}
+
 /* ggdmc_loglike and its allocation-free variant: the design, trials, thetas
  * and output are packed into one device buffer, allocated per call or (noalloc)
  * the device's staging array, the only difference between the two. */
@@ -1395,22 +1444,25 @@ static int loglike_impl(const ggdmc_model *model, const ggdmc_subject *data, con
             for (int64_t i = data->cell_off[c]; i < data->cell_off[c + 1]; ++i)
                 tcode[i] = (uint16_t)((cond.cond_of_cell[c] << 3) | model->winner[c]);
         const int nq = cond.n_cond;
-        const int64_t soff[2] = {0, T};
         auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
         const size_t o_src = 0, o_const = o_src + al(sizeof(int32_t) * nq * na * 6);
         const size_t o_rt = o_const + al(sizeof(double) * nq * na * 6);
         const size_t o_cell = o_rt + al(sizeof(double) * (size_t)T);
-        const size_t o_off = o_cell + al(sizeof(uint16_t) * (size_t)T);
-        const size_t o_tab = o_off + al(sizeof(soff));
+        const size_t o_tab = o_cell + al(sizeof(uint16_t) * (size_t)T);
         const size_t o_th = o_tab + al(sizeof(double) * 64);
-        const size_t o_out = o_th + al(sizeof(double) * (size_t)n * P);
-        const size_t total = o_out + al(sizeof(double) * (size_t)n);
-        std::vector<char> h(total);
+        const size_t o_ctr = o_th + al(sizeof(double) * (size_t)n * P);
+        LoglikeSplit sp = loglike_split(n, T, nq * na, P, true);
+        auto sums = [&]() { return sp.nsplit > 1 ? al(sizeof(double) * (size_t)n * sp.nj) : (size_t)0; };
+        auto ctrs = [&]() { return sp.nsplit > 1 ? al(sizeof(uint32_t) * (size_t)((n + sp.k - 1) / sp.k)) : al(1); };
+        const size_t n_out = al(sizeof(double) * (size_t)n);
+        /* a call that fits the fixed array without chunk sums is not refused for them */
+        if (noalloc && o_ctr + ctrs() + n_out + sums() > kStagingBytes) sp = loglike_split(n, T, nq * na, P, false);
+        const size_t o_out = o_ctr + ctrs(), o_sum = o_out + n_out, total = o_sum + sums();
+        std::vector<char> h(o_out);   /* uploaded; counters are zero */
         std::memcpy(&h[o_src], cond.src.data(), sizeof(int32_t) * nq * na * 6);
         std::memcpy(&h[o_const], cond.cst.data(), sizeof(double) * nq * na * 6);
         if (T) std::memcpy(&h[o_rt], data->rt, sizeof(double) * (size_t)T);
         if (T) std::memcpy(&h[o_cell], tcode.data(), sizeof(uint16_t) * (size_t)T);
-        std::memcpy(&h[o_off], soff, sizeof(soff));
         fill_exp2_table(reinterpret_cast<double *>(&h[o_tab]));
         std::memcpy(&h[o_th], theta, sizeof(double) * (size_t)n * P);
         char *b = nullptr;
@@ -1436,13 +1488,12 @@ static int loglike_impl(const ggdmc_model *model, const ggdmc_subject *data, con
         d.par_const = reinterpret_cast<const double *>(b + o_const);
         d.rt = reinterpret_cast<const double *>(b + o_rt);
         d.tcode = reinterpret_cast<const uint16_t *>(b + o_cell);
-        d.subj_off = reinterpret_cast<const int64_t *>(b + o_off);
         d.exp2tab = reinterpret_cast<const double *>(b + o_tab);
         d.S = 1;
-        const int cmax = (int)std::max<int64_t>(1, std::min<int64_t>((T + kChunk - 1) / kChunk, 1024));
-        const size_t lds = ggdmc_internal_sweep_lds(1, P, 1, nq * na, 1, cmax, 0);
-        HIPCHECK(ggdmc_internal_launch_loglike(&d, reinterpret_cast<const double *>(b + o_th), n, 0,
-                                               precision, cmax, lds, nullptr,
+        const size_t lds = ggdmc_internal_sweep_lds(1, P, sp.k, nq * na, sp.k, sp.cmax, sp.tstage);
+        HIPCHECK(ggdmc_internal_launch_loglike(&d, &sp, reinterpret_cast<const double *>(b + o_th), precision, lds,
+                                               nullptr, reinterpret_cast<double *>(b + o_sum),
+                                               reinterpret_cast<uint32_t *>(b + o_ctr),
                                                reinterpret_cast<double *>(b + o_out)));
         HIPCHECK(hipMemcpy(ll_out, b + o_out, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost));
         if (dbuf) HIPCHECK(hipFree(dbuf));

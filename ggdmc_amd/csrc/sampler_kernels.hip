@@ -2272,25 +2272,107 @@ __global__ void hyper_data_stats_kernel(Dev d, const double *rows, int S, int f)
 }
 
 /* ----------------------------------------------------------- sumloglike */
-/* out[q] = log-likelihood of thetas[q] over subject s's trials, with the
- * sampler's canonical chunk sums (bit-identical to the sampler's values). */
+/* s + t[0] + .. + t[m-1], added in order; eight loads in flight. */
+__device__ __forceinline__ double ordered_sum(double s, const double *t, int m) {
+    int j = 0;
+    for (; j + 8 <= m; j += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = t[j + u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; j < m; ++j) s += t[j];
+    return s;
+}
+
+/* out[q] = log-likelihood of thetas[q] over the trials, with the sampler's
+ * canonical chunk sums (bit-identical to the sampler's values). A workgroup
+ * takes sp.k vectors and sp.jper chunks; with several workgroups per vector the
+ * chunk sums meet in csum ([vector][chunk]) and the last-arriving workgroup of
+ * the vectors adds them in order (device-scope stores complete before the
+ * counter, device-scope loads after it, as the sweep kernel's tiles).
+ *
+ * What bounds it is the constants' set-up (one thread per condition and
+ * accumulator: three divisions and a normal tail in a row, about 4 us, during
+ * which the workgroup's other waves have nothing to do), the number of waves
+ * that have trials, and for large calls vector issue. The split (loglike_split
+ * in engine.hip) follows those. */
 template <int MODE>
-__global__ __launch_bounds__(kBlock) void loglike_kernel(Dev d, const double *thetas, int s, int cmax,
-                                                        double *out) {
+__global__ __launch_bounds__(kLoglikeBlock) void loglike_kernel(Dev d, LoglikeSplit sp, const double *thetas,
+                                                                double *csum, uint32_t *ctr, double *out) {
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
-    const int P = d.P;
-    const SweepLds L = carve(lds_raw, 1, P, 1, d.n_cond * d.n_acc, 1, cmax, 0);
-    const int q = blockIdx.x;
-    load_exp2_table(d);
-    for (int p = threadIdx.x; p < P; p += blockDim.x) L.prop[p] = thetas[(size_t)q * P + p];
-    stage_copy(L.psrc, d.par_src, d.n_cond * d.n_acc * 6);
-    stage_copy(L.pcst, d.par_const, d.n_cond * d.n_acc * 6);
-    if (threadIdx.x == 0) L.active[0] = 1;
+    const int P = d.P, per = d.n_cond * d.n_acc;
+    const SweepLds L = carve(lds_raw, 1, P, sp.k, per, sp.k, sp.cmax, sp.tstage);
+    const int blk = (int)blockIdx.x / sp.nsplit, part = (int)blockIdx.x - blk * sp.nsplit;
+    const int q0 = blk * sp.k, kb = min(sp.k, sp.n - q0);
+    const int j0 = part * sp.jper, j1 = min(sp.nj, j0 + sp.jper);
+    const int64_t t_lo = (int64_t)j0 * kChunk, t_hi = min(sp.ntrial, (int64_t)j1 * kChunk);
+    const int nst = sp.tstage > 0 ? (int)(t_hi - t_lo) : 0;
+    {
+        /* every load of the set-up in flight together */
+        Piece<double, 1> pex{g_exp2tab, d.exp2tab, 64};
+        Piece<double, 1> pth{L.prop, thetas + (size_t)q0 * P, kb * P};
+        Piece<int32_t, 1> psr{L.psrc, d.par_src, per * 6};
+        Piece<double, 1> pcs{L.pcst, d.par_const, per * 6};
+        Piece<double, 4> prt{L.trt, d.rt + t_lo, nst};
+        Piece<uint16_t, 4> pcd{L.tcd, d.tcode + t_lo, nst};
+        pex.load();
+        pth.load();
+        psr.load();
+        pcs.load();
+        prt.load();
+        pcd.load();
+        pex.store();
+        pth.store();
+        psr.store();
+        pcs.store();
+        prt.store();
+        pcd.store();
+    }
+    for (int c = threadIdx.x; c < kb; c += blockDim.x) {
+        L.active[c] = 1;
+        L.tll[c] = 0.0;
+    }
+    const TrialView tv = nst > 0 ? TrialView{L.trt, L.tcd, t_lo} : TrialView{d.rt, d.tcode, 0};
     __syncthreads();
-    const int64_t t0 = d.subj_off[s], t1 = d.subj_off[s + 1];
-    const int nj = (int)((t1 - t0 + kChunk - 1) / kChunk);
-    proposals_loglike<MODE>(d, L, TrialView{d.rt, d.tcode, 0}, 1, 1, cmax, t0, t1, 0, nj, false, 0, 0);
-    if (threadIdx.x == 0) out[q] = L.tll[0];
+    build_acck(d, L, L.prop, P, 0, kb, L.acck);
+    __syncthreads();
+    for (int jb = j0; jb < j1; jb += sp.cmax) {
+        const int nbat = min(sp.cmax, j1 - jb);
+        chunk_sums<MODE>(d, tv, 0, sp.ntrial, jb, nbat, kb, L.active, L.acck, L.csum, sp.cmax, L.pend);
+        __syncthreads();
+        if (sp.nsplit > 1) {
+            for (int e = threadIdx.x; e < kb * nbat; e += blockDim.x) {
+                const int c = e / nbat, jj = e - c * nbat;
+                __hip_atomic_store(csum + (size_t)(q0 + c) * sp.nj + jb + jj, L.csum[(size_t)c * sp.cmax + jj],
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        } else {
+            for (int c = threadIdx.x; c < kb; c += blockDim.x)
+                L.tll[c] = ordered_sum(L.tll[c], L.csum + (size_t)c * sp.cmax, nbat);
+        }
+        __syncthreads();
+    }
+    if (sp.nsplit > 1) {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        if (threadIdx.x == 0) L.flag[0] = atomicAdd(ctr + blk, 1u) == (uint32_t)(sp.nsplit - 1);
+        __syncthreads();
+        if (!L.flag[0]) return;
+        for (int jb = 0; jb < sp.nj; jb += sp.cmax) {
+            const int nbat = min(sp.cmax, sp.nj - jb);
+            for (int e = threadIdx.x; e < kb * nbat; e += blockDim.x) {
+                const int c = e / nbat, jj = e - c * nbat;
+                L.csum[(size_t)c * sp.cmax + jj] = ld<true>(csum + (size_t)(q0 + c) * sp.nj + jb + jj);
+            }
+            __syncthreads();
+            for (int c = threadIdx.x; c < kb; c += blockDim.x)
+                L.tll[c] = ordered_sum(L.tll[c], L.csum + (size_t)c * sp.cmax, nbat);
+            __syncthreads();
+        }
+    }
+    for (int c = threadIdx.x; c < kb; c += blockDim.x) out[q0 + c] = L.tll[c];
 }
 
 } // namespace ggdmc
@@ -2373,13 +2455,14 @@ hipError_t ggdmc_internal_launch_hyper_stats(const Dev *d, const double *rows, i
     return hipGetLastError();
 }
 
-hipError_t ggdmc_internal_launch_loglike(const Dev *d, const double *thetas, int nq, int s,
-                                         int mode, int cmax, size_t lds, hipStream_t stream,
+hipError_t ggdmc_internal_launch_loglike(const Dev *d, const LoglikeSplit *sp, const double *thetas, int mode,
+                                         size_t lds, hipStream_t stream, double *csum, uint32_t *ctr,
                                          double *out) {
+    const dim3 grid((unsigned)(((sp->n + sp->k - 1) / sp->k) * sp->nsplit)), block(sp->threads);
     if (mode == GGDMC_MIXED_BATCHED)
-        loglike_kernel<MODE_MIXED><<<dim3(nq), dim3(kBlock), lds, stream>>>(*d, thetas, s, cmax, out);
+        loglike_kernel<MODE_MIXED><<<grid, block, lds, stream>>>(*d, *sp, thetas, csum, ctr, out);
     else
-        loglike_kernel<MODE_NAIVE><<<dim3(nq), dim3(kBlock), lds, stream>>>(*d, thetas, s, cmax, out);
+        loglike_kernel<MODE_NAIVE><<<grid, block, lds, stream>>>(*d, *sp, thetas, csum, ctr, out);
     return hipGetLastError();
 }
 
