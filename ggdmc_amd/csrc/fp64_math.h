@@ -70,8 +70,9 @@ constexpr double kMillsPieces[9][17] = {
 constexpr double kLn2By64Hi = 0.010830424696249145, kLn2By64Lo = 3.623510646634843e-19;
 constexpr double kLn2Hi = 0.6931471805599453, kLn2Lo = 2.3190468138462996e-17;
 
-/* e^x; x > 709.78 overflows to +inf, x < -745.2 underflows to 0, NaN passes. */
-GGDMC_MFN double exp_acc(double x) {
+/* e^x; x > 709.78 overflows to +inf, x < -745.2 underflows to 0, NaN passes.
+ * tab: the 64 values above or a copy of them. */
+GGDMC_MFN double exp_acc(double x, const double *tab = kExp2Tab) {
     const bool in = x > -745.2 && x < 709.8;
     const double xc = in ? x : 0.0;
     const double k = std::rint(xc * 92.33248261689366);   /* 64 / ln 2 */
@@ -82,7 +83,7 @@ GGDMC_MFN double exp_acc(double x) {
                                          r * (0.041666666666666664 +
                                               r * (0.008333333333333333 + r * 0.001388888888888889)))));
     const int ki = (int)k;
-    const double v = std::ldexp(kExp2Tab[ki & 63] * p, ki >> 6);
+    const double v = std::ldexp(tab[ki & 63] * p, ki >> 6);
     return in ? v : (x != x ? x : (x > 0.0 ? HUGE_VAL : 0.0));
 }
 
@@ -113,29 +114,57 @@ GGDMC_MFN double log_acc(double x) {
     return finite ? v : (x == 0.0 ? -HUGE_VAL : (x == HUGE_VAL ? x : (x - x) / 0.0 * 0.0 + NAN));
 }
 
-/* The Mills ratio R(a) = Q(a) exp(a^2/2), a >= 0. */
-GGDMC_MFN double mills_acc(double a) {
+/* The Mills ratio R(a) = Q(a) exp(a^2/2), a >= 0. pieces: kMillsPieces or a
+ * copy. The asymptotic piece and its two divisions stand behind a branch that
+ * few waves take. */
+GGDMC_MFN double mills_acc(double a, const double *pieces = &kMillsPieces[0][0]) {
     const int k = a < 8.0 ? (int)a : 8;
-    const double s = a < 8.0 ? 2.0 * (a - (double)k) - 1.0 : 128.0 / (a * a) - 1.0;
-    const double *c = kMillsPieces[k];
+    double s = 2.0 * (a - (double)k) - 1.0;
+    if (!(a < 8.0)) s = 128.0 / (a * a) - 1.0;
+    const double *c = pieces + k * (kMillsPieceDeg + 1);
     double h = c[kMillsPieceDeg];
+#pragma unroll
     for (int j = kMillsPieceDeg - 1; j >= 0; --j) h = c[j] + s * h;
-    return a < 8.0 ? h : h / a;
+    if (!(a < 8.0)) h = h / a;
+    return h;
 }
 
 /* Q(a) = P(Z > a) for a >= 0 (a = +inf gives 0, NaN passes). */
-GGDMC_MFN double qtail_acc(double a) {
+GGDMC_MFN double qtail_acc(double a, const double *tab = kExp2Tab, const double *pieces = &kMillsPieces[0][0]) {
     if (!(a < 1e300)) return a != a ? a : 0.0;
     const double a2 = a * a;
     const double a2l = std::fma(a, a, -a2);         /* a^2 = a2 + a2l exactly */
-    const double e = exp_acc(-0.5 * a2);
-    return std::fma(e, -0.5 * a2l, e) * mills_acc(a);
+    const double e = exp_acc(-0.5 * a2, tab);
+    return std::fma(e, -0.5 * a2l, e) * mills_acc(a, pieces);
 }
 
 /* Phi(z) as R's pnorm rounds it: the lower tail directly, above 0 as
  * 1 - the upper tail. */
 GGDMC_MFN double pnorm_acc(double z) {
     return z > 0.0 ? 1.0 - qtail_acc(z) : qtail_acc(-z);
+}
+
+/* P = pnorm_acc(z) and e = exp_acc(-z^2/2), the same bits from one exponential
+ * (z^2/2 is the argument of both) and without the range selects that a
+ * non-positive argument does not need: |z| is cut at 40, where Q is 0. A NaN z
+ * gives a NaN P (through the Mills ratio). */
+GGDMC_MFN void normal_acc(double z, const double *tab, const double *pieces, double &P, double &e) {
+    double a = std::fabs(z);
+    a = a > 40.0 ? 40.0 : a;
+    const double a2 = a * a;
+    const double a2l = std::fma(a, a, -a2);
+    const double x = -0.5 * a2;
+    const double k = std::rint(x * 92.33248261689366);   /* 64 / ln 2 */
+    double r = std::fma(-k, kLn2By64Hi, x);
+    r = std::fma(-k, kLn2By64Lo, r);
+    const double p =
+        1.0 + r * (1.0 + r * (0.5 + r * (0.16666666666666666 +
+                                         r * (0.041666666666666664 +
+                                              r * (0.008333333333333333 + r * 0.001388888888888889)))));
+    const int ki = (int)k;
+    e = std::ldexp(tab[ki & 63] * p, ki >> 6);
+    const double q = std::fma(e, -0.5 * a2l, e) * mills_acc(a, pieces);
+    P = z > 0.0 ? 1.0 - q : q;
 }
 
 } // namespace ggdmc

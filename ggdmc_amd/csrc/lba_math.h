@@ -248,21 +248,76 @@ GGDMC_FN Core mixed_core(const AccK &k, double t) {
 }
 
 /* ------------------------------------------------------------- naive FP64 */
+/* P = Phi(z) and d = phi(z): in one step where Ops has one (the kernels: the
+ * same bits, from tables in LDS). */
+template <class Ops>
+GGDMC_FN auto normal_parts(double z, double &P, double &d, int) -> decltype(Ops::normal(z, P, d)) {
+    Ops::normal(z, P, d);
+}
+template <class Ops>
+GGDMC_FN void normal_parts(double z, double &P, double &d, long) {
+    P = Ops::pnorm(z);
+    d = Ops::dnorm(z);
+}
+
+/* x / d correctly rounded for finite x, y = 1/d correctly rounded: q = x*y,
+ * then r = x - q*d exactly (one FMA) and RN(q + r*y) = RN(x/d) (Markstein's
+ * correction step), while nothing overflows and x is 0 or above 1e-290. */
+GGDMC_FN double div_finite(double x, double d, double y) {
+    const double q = x * y;
+    return std::fma(std::fma(-q, d, x), y, q);
+}
+
+/* The reference's intermediate values of one accumulator at t > 0. The two
+ * quotients by zs share one division and correct its reciprocal (the same bits
+ * as two divisions, of about 15 issue slots each); fine: the operands lie where
+ * that holds (a quotient that the correction could round differently is below
+ * 1e-190). */
+struct NaiveParts {
+    double zs, chi, chimA, P1, P2, d1, d2;
+    bool fine;
+};
+
+template <class Ops>
+GGDMC_FN NaiveParts naive_parts(const AccK &k, double t) {
+    NaiveParts n;
+    n.zs = t * k.s;
+    n.chi = k.b - t * k.v;
+    n.chimA = n.chi - k.A;
+    n.fine = k.eL == k.eL && n.zs > 1e-100 && n.zs < 1e100 && std::fabs(n.chi) < 1e100;
+    const double y = 1.0 / n.zs;
+    double z1 = div_finite(n.chi, n.zs, y), z2 = div_finite(n.chimA, n.zs, y);
+    if (__builtin_expect(!n.fine, 0)) {
+        z1 = n.chi / n.zs;
+        z2 = n.chimA / n.zs;
+    }
+    normal_parts<Ops>(z1, n.P1, n.d1, 0);
+    normal_parts<Ops>(z2, n.P2, n.d2, 0);
+    return n;
+}
+
+template <class Ops>
+GGDMC_FN double naive_pdf(const AccK &k, double t) {
+    if (!(t > 0.0)) return t == t ? 0.0 : t;
+    const NaiveParts n = naive_parts<Ops>(k, t);
+    return (k.v * (n.P1 - n.P2) + k.s * (n.d2 - n.d1)) / (k.A * k.den);
+}
+
+template <class Ops>
+GGDMC_FN double naive_cdf(const AccK &k, double t) {
+    if (!(t > 0.0)) return t == t ? 0.0 : t;
+    const NaiveParts n = naive_parts<Ops>(k, t);
+    const double num = n.zs * (n.d2 - n.d1) + n.chimA * n.P2 - n.chi * n.P1;
+    /* quotients by A and den from their stored reciprocals */
+    double cdf = div_finite(1.0 + div_finite(num, k.A, k.invA), k.den, k.inv_den);
+    if (__builtin_expect(!n.fine, 0)) cdf = (1.0 + num / k.A) / k.den;
+    return cdf;
+}
+
 template <class Ops>
 GGDMC_FN void naive_pdf_cdf(const AccK &k, double t, double &pdf, double &cdf) {
-    if (!(t > 0.0)) {
-        pdf = t == t ? 0.0 : t;
-        cdf = pdf;
-        return;
-    }
-    const double zs = t * k.s;
-    const double chi = k.b - t * k.v;
-    const double chimA = chi - k.A;
-    const double z1 = chi / zs, z2 = chimA / zs;
-    const double P1 = Ops::pnorm(z1), P2 = Ops::pnorm(z2);
-    const double d1 = Ops::dnorm(z1), d2 = Ops::dnorm(z2);
-    pdf = (k.v * (P1 - P2) + k.s * (d2 - d1)) / (k.A * k.den);
-    cdf = (1.0 + (zs * (d2 - d1) + chimA * P2 - chi * P1) / k.A) / k.den;
+    pdf = naive_pdf<Ops>(k, t);
+    cdf = naive_cdf<Ops>(k, t);
 }
 
 /* Error model of the mixed evaluation: every computed tail and exp(-z^2/2)
@@ -279,14 +334,9 @@ constexpr double kUlp1 = 1.1102230246251565e-16;
 /* a loser's reference noise per unit of D1 + D2 > K (|chi| + |chi - A|) */
 constexpr double kLoserUlp = 4.3e-16; /* above kUlp1 / kMillsK */
 
-/* x / d correctly rounded, given y = 1/d correctly rounded: q = x*y, then
- * r = x - q*d exactly (one FMA) and RN(q + r*y) = RN(x/d) (Markstein's
- * correction step) for finite x; x = +-inf takes x*y, which is x/d there.
- * Three FP64 operations instead of a division sequence. */
+/* div_finite for any x: x = +-inf takes x*y, which is x/d there. */
 GGDMC_FN double div_rn(double x, double d, double y) {
-    const double q = x * y;
-    const double c = std::fma(std::fma(-q, d, x), y, q);
-    return std::isinf(x) ? q : c;
+    return std::isinf(x) ? x * y : div_finite(x, d, y);
 }
 
 /* One accumulator of a trial: its factor of the density, and whether the quick
@@ -387,10 +437,7 @@ GGDMC_FN Factor loser_factor(const AccK &k, double rt) {
     f.c = mixed_core<Ops>(k, f.t);
     const double P2 = (f.c.z2 < 0.0 ? 0.0 : 1.0) - f.c.a2;
     f.num = std::fma(std::fma(-kInvSqrt2Pi, f.c.zs * f.c.de, f.c.chi * f.c.dP), k.invA, P2); /* 1 - G */
-    /* RN((1 - (1 - G)) / den), as div_rn */
-    const double x = 1.0 - f.num;
-    const double y = x * k.inv_den;
-    const double F = std::fma(std::fma(-y, k.den, x), k.inv_den, y);
+    const double F = div_finite(1.0 - f.num, k.den, k.inv_den);
     f.val = 1.0 - std::fmax(or_negative(F, f.pos), kFloor);
     f.ok = std::fma(f.c.zs, 0.345e-9 / kLoserUlp, f.c.D) * k.eL <= std::fabs(f.val);
     return f;
@@ -444,14 +491,13 @@ GGDMC_FN double mixed_loser_survivor(const AccK &k, double rt, bool &ill) {
  * the batched path's ill-conditioned trials. */
 template <class Ops>
 GGDMC_FN double naive_trial_term(const AccK *kc, int n_acc, int w, double rt) {
-    double pdf, cdf;
-    naive_pdf_cdf<Ops>(kc[w], rt - kc[w].t0, pdf, cdf);
+    const double pdf = naive_pdf<Ops>(kc[w], rt - kc[w].t0);
     double dens = pdf != pdf ? pdf : (pdf > kFloor ? pdf : kFloor);
     /* losers in accumulator order; indexing the l-th loser (rather than
      * skipping j == w) keeps every lane of a wave on the same iteration */
     for (int l = 0; l + 1 < n_acc; ++l) {
         const int j = l + (l >= w);
-        naive_pdf_cdf<Ops>(kc[j], rt - kc[j].t0, pdf, cdf);
+        const double cdf = naive_cdf<Ops>(kc[j], rt - kc[j].t0);
         const double F = cdf != cdf ? cdf : (cdf > kFloor ? cdf : kFloor);
         dens *= (1.0 - F);
     }

