@@ -112,6 +112,18 @@ struct Pool {
     }
 };
 
+/* A HIP event for one scope. */
+struct Event {
+    hipEvent_t e = nullptr;
+    hipEvent_t get() {
+        if (!e) HIPCHECK(hipEventCreate(&e));
+        return e;
+    }
+    ~Event() {
+        if (e) (void)hipEventDestroy(e);
+    }
+};
+
 int device_cus() {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
@@ -153,6 +165,8 @@ struct ggdmc_session {
     int kmax = 1, cmax = 1, chain_batch = 1, tstage = 0;
     std::vector<const int4 *> lists;   /* item list per launch (per group, or one) */
     std::vector<int> list_n;
+    int4 *list_mem = nullptr;          /* the lists' memory, reused by the next decomposition */
+    size_t list_cap = 0;
     size_t sweep_lds = 0, phi_lds = 0;
     int phi_stats_lds = 0;        /* population kernel keeps the statistics in LDS */
     /* population step inside the subject launches (leading workgroups of
@@ -173,6 +187,7 @@ struct ggdmc_session {
     uint32_t next_iter = 1;      /* next local iteration to run (1-based) */
     uint32_t last_iter = 0;      /* nmc*thin - 1 */
     uint32_t *iter_base = nullptr;
+    uint32_t base_now = UINT32_MAX;   /* value last written to iter_base */
     hipGraphExec_t graph = nullptr;
     int graph_iters = 0;
     /* a graph of the remainder of the last advance (fewer iterations than
@@ -205,10 +220,27 @@ struct ggdmc_session {
     void set_decomp(bool fused_new, int k_new, int tpt_new, bool chained_new = false, int ipl_new = 1,
                     bool span_new = false, int occ_new = 3);
     void default_decomp();
+    /* a work decomposition of the subject launches */
+    struct Decomp {
+        bool fused;
+        int k, tpt;
+        bool chained;
+        int ipl;
+        bool span;
+        int occ;
+    };
+    std::vector<Decomp> candidates() const;
+    bool try_decomp(const Decomp &c);
+    bool decomp_given() const {
+        return cfg.trials_per_tile != 0 || cfg.chains_per_item != 0 || cfg.launch_mode >= 2;
+    }
     void enqueue_iteration(uint32_t off, std::vector<hipEvent_t> *ev = nullptr, int count = 1);
     void flush_store();
+    void set_base(uint32_t v);
     void run_batched(uint32_t n_iter);
     void run_plain(uint32_t n_iter);
+    void run_whole();
+    void run_timed(uint32_t n_iter, bool whole);
     void autotune();
     void capture(int K);
     hipGraphExec_t make_graph(int K);
@@ -559,6 +591,14 @@ void ggdmc_session::build(const ggdmc_config *c, const ggdmc_model *model, const
     }
     iter_base = pool.alloc<uint32_t>(1);
     d.iter_base = iter_base;
+    {
+        /* flags and counters of every decomposition: at most one chain range
+         * per chain of a group */
+        const size_t nf = (size_t)std::max(S, 1) * G * ((n + G - 1) / G);
+        d.item_ready = pool.alloc<uint32_t>(nf);
+        d.item_staged = pool.alloc<uint32_t>(nf);
+        d.tile_ctr = pool.alloc<uint32_t>(nf);
+    }
     hyper_rows = pool.upload(hyper_rows_h, stream);
     hyper_off = pool.upload(hyper_off_h, stream);
 
@@ -655,7 +695,7 @@ void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chai
     list_n.clear();
     int64_t max_chunks_item = 1;
     const int nl = (fused || span) ? 1 : G;
-    std::vector<int4> all_items;   /* every group's items, in group order (chained) */
+    std::vector<int4> all_items;   /* every group's items, in group order */
     rmax = 1;
     /* XCD-aware order: workgroup w runs on XCD w % 8, so the items of subject
      * x go to workgroups w = x (mod 8) where possible, and share that XCD's
@@ -708,24 +748,32 @@ void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chai
             continue;
         }
         xcd_order(items, phi_in ? (int64_t)d.n_phi * ng : 0);
-        require(items.size() < ((size_t)1 << 31), "too many work items");
+        all_items.insert(all_items.end(), items.begin(), items.end());
         list_n.push_back((int)items.size());
-        lists.push_back(pool.upload(items, stream));
     }
-    if (chained) {
-        require(all_items.size() < ((size_t)1 << 31), "too many work items");
-        list_n.push_back((int)all_items.size());
-        lists.push_back(pool.upload(all_items, stream));
-        const size_t nf = (size_t)std::max(d.S, 1) * G * rmax;
-        d.item_ready = pool.alloc<uint32_t>(nf);
-        HIPCHECK(hipMemsetAsync(d.item_ready, 0, sizeof(uint32_t) * nf, stream));
-        d.item_staged = pool.alloc<uint32_t>(nf);
-        HIPCHECK(hipMemsetAsync(d.item_staged, 0, sizeof(uint32_t) * nf, stream));
+    require(all_items.size() < ((size_t)1 << 31), "too many work items");
+    if (chained) list_n.push_back((int)all_items.size());
+    if (all_items.size() > list_cap) {
+        list_mem = pool.alloc<int4>(all_items.size());
+        list_cap = all_items.size();
+    }
+    if (!all_items.empty()) {
+        /* launches still running may read the lists: stream order, and the
+         * host vector lives until the copy is done */
+        HIPCHECK(hipMemcpyAsync(list_mem, all_items.data(), sizeof(int4) * all_items.size(), hipMemcpyHostToDevice,
+                                stream));
+        HIPCHECK(hipStreamSynchronize(stream));
+    }
+    size_t first = 0;
+    for (const int m : list_n) {
+        lists.push_back(list_mem + first);
+        first += (size_t)m;
     }
     {
-        const size_t nctr = (size_t)std::max(d.S, 1) * G * rmax;
-        d.tile_ctr = pool.alloc<uint32_t>(nctr);
-        HIPCHECK(hipMemsetAsync(d.tile_ctr, 0, sizeof(uint32_t) * nctr, stream));
+        const size_t nf = (size_t)std::max(d.S, 1) * G * rmax;
+        HIPCHECK(hipMemsetAsync(d.item_ready, 0, sizeof(uint32_t) * nf, stream));
+        HIPCHECK(hipMemsetAsync(d.item_staged, 0, sizeof(uint32_t) * nf, stream));
+        HIPCHECK(hipMemsetAsync(d.tile_ctr, 0, sizeof(uint32_t) * nf, stream));
     }
     /* LDS: accumulator constants of chain_batch chains and cmax chunk sums
      * per chain at once, within 48 KB when possible */
@@ -860,29 +908,35 @@ void ggdmc_session::prepare_rest(uint32_t n_iter) {
     rest_iters = r;
 }
 
+void ggdmc_session::set_base(uint32_t v) {
+    if (base_now == v) return;
+    set_base_kernel<<<1, 1, 0, stream>>>(iter_base, v);
+    HIPCHECK(hipGetLastError());
+    base_now = v;
+}
+
+/* Graph replays take their first iteration from the device word; launches
+ * outside a graph carry it in their arguments (base 0), without a kernel to
+ * write it before each. */
 void ggdmc_session::run_batched(uint32_t n_iter) {
     if (n_iter == 0) return;
     while (n_iter > 0) {
+        uint32_t cnt;
         if (graph && n_iter >= (uint32_t)graph_iters) {
-            set_base_kernel<<<1, 1, 0, stream>>>(iter_base, next_iter);
-            HIPCHECK(hipGetLastError());
+            set_base(next_iter);
             HIPCHECK(hipGraphLaunch(graph, stream));
-            next_iter += graph_iters;
-            n_iter -= graph_iters;
+            cnt = (uint32_t)graph_iters;
         } else if (rest_graph && n_iter == (uint32_t)rest_iters) {
-            set_base_kernel<<<1, 1, 0, stream>>>(iter_base, next_iter);
-            HIPCHECK(hipGetLastError());
+            set_base(next_iter);
             HIPCHECK(hipGraphLaunch(rest_graph, stream));
-            next_iter += rest_iters;
-            n_iter = 0;
+            cnt = (uint32_t)rest_iters;
         } else {
-            set_base_kernel<<<1, 1, 0, stream>>>(iter_base, next_iter);
-            HIPCHECK(hipGetLastError());
-            const int cnt = (int)std::min<uint32_t>(chained ? (uint32_t)ipl : 1u, n_iter);
-            enqueue_iteration(0, nullptr, cnt);
-            next_iter += (uint32_t)cnt;
-            n_iter -= (uint32_t)cnt;
+            set_base(0);
+            cnt = std::min<uint32_t>(chained ? (uint32_t)ipl : 1u, n_iter);
+            enqueue_iteration(next_iter, nullptr, (int)cnt);
         }
+        next_iter += cnt;
+        n_iter -= cnt;
     }
     flush_store();
 }
@@ -905,46 +959,180 @@ void ggdmc_session::run_plain(uint32_t n_iter) {
     }
 }
 
-/* Picks the work decomposition by timing graph replays of a few real
+bool ggdmc_session::try_decomp(const Decomp &c) {
+    try {
+        set_decomp(c.fused, c.k, c.tpt, c.chained, c.ipl, c.span, c.occ);
+    } catch (const Error &) {
+        if (c.ipl == 1) throw;
+        return false;   /* no population step inside the launch for this design */
+    }
+    return true;
+}
+
+/* Decompositions worth timing, the likeliest first. With whole subjects and
+ * several iterations per launch an iteration costs the same set-up, waits and
+ * likelihood phases whatever k, so an item should hold as few chains as still
+ * fit on the chip together: workgroups are resident 3 to a CU with the 3-wave
+ * build (4 with the 4-wave one), and items beyond that wait for a round of
+ * their own. Measured (us an iteration, k = 1, 2, 4, 8, all chains of a group):
+ *   32 x 768, 20 chains a group (640 items at k = 1): 35, 37, 47, 69, 150
+ *   100 x 550, 20 chains (500 at k = 4): 93, 61, 46, 66, 136
+ *   64 x 1000 of 4 accumulators, 17 chains (576 at k = 2): 70, 57, 84, 134, 241
+ *   320 x 96..2048 with 4 waves (1600 at k = 4): 279, 196, 160, 176, 403
+ *   512 x 768 with 4 waves (1536 at k = 8): 394, 248, 185, 170, 192
+ *   1024 x 2048 of 4 accumulators (1024 with all): -, 1209, 1074, 1068, 999
+ * So: all chains of a group when the subjects alone fill the chip; else the
+ * smallest k that keeps 3 items a CU, while that is at most 4; else the smallest
+ * k from 4 that keeps 6.25 a CU, with 4 waves. The first candidate is within 13 %
+ * of the best of about 45 on 20 workloads, and one of the list is the best or
+ * within 3 % of it: its neighbours in k, launch mode and build follow, and trial
+ * tiles where few long subjects leave the chip idle (1 x 4096, 18 chains: tiles
+ * of 256 41 us, whole subjects 50). */
+std::vector<ggdmc_session::Decomp> ggdmc_session::candidates() const {
+    const int ng = (d.nchain + d.G - 1) / d.G;
+    const int64_t cus = std::max(device_cus(), 1);
+    std::vector<int> ks;
+    for (int k : {1, 2, 4, 8, ng})
+        if (k <= ng && std::find(ks.begin(), ks.end(), k) == ks.end()) ks.push_back(k);
+    auto items = [&](int k) { return (int64_t)d.S * ((ng + k - 1) / k); };
+    auto smallest = [&](int64_t most) {
+        size_t i = 0;
+        while (i + 1 < ks.size() && items(ks[i]) > most) ++i;
+        return i;
+    };
+    size_t i = smallest(3 * cus);
+    int occ = 3;
+    if (d.S < 3 * cus && ks[i] > 4) {
+        i = std::max(smallest(25 * cus / 4), (size_t)2);
+        occ = 4;
+    }
+    const int k = ks[i];
+    std::vector<Decomp> out;
+    auto add = [&](const Decomp &c) {
+        for (const Decomp &o : out)
+            if (o.fused == c.fused && o.k == c.k && o.tpt == c.tpt && o.chained == c.chained && o.ipl == c.ipl &&
+                o.span == c.span && o.occ == c.occ)
+                return;
+        out.push_back(c);
+    };
+    /* several iterations per launch wait for each other's items a bounded time
+     * (kSpinLimit polls, about 0.4 s): an item's likelihoods, or a migration
+     * ring's, must stay far below it. A chunk of a chain takes a wave about 4 us
+     * with 2 accumulators, three times that in FP64. */
+    const double chunk_us = 2.0 * d.n_acc * (mode == GGDMC_FP64_BATCHED ? 3.0 : 1.0);
+    const double rounds = std::ceil((double)max_ntr / kChunk / kWaves);
+    const bool can_chain = nsweep_sub == 1 && cfg.launch_mode != 1 &&
+                           rounds * chunk_us * std::max(k, d.sub_mig > 0.0 ? d.nchain : 1) < 5e4;
+    if (can_chain) {
+        auto multi = [&](int kk, bool span, int oc) {
+            if (cfg.waves_per_simd != 0) oc = cfg.waves_per_simd;
+            if (span && !span_fits((ng + kk - 1) / kk)) span = false;
+            add({false, kk, 0, true, kItersPerLaunch, span, oc});
+        };
+        const bool span = k == 1 || k == ng;
+        if (items(1) <= cus && max_ntr >= 2048) {
+            add({false, std::min(2, ng), 256, true, 1, false, 3});
+            add({false, 1, 256, true, 1, false, 3});
+        }
+        multi(k, span, occ);
+        if (d.G > 2) add({true, 0, 0, false, 1, false, 3});
+        multi(k, !span, occ);
+        multi(k, span, 7 - occ);
+        if (i + 1 < ks.size()) multi(ks[i + 1], false, 3);
+        if (i > 0) multi(ks[i - 1], false, 4);
+        if (i > 0) multi(ks[i - 1], true, 4);
+        if (items(1) <= cus && max_ntr > 1024) add({false, 1, 1024, true, 1, false, 3});
+        add({false, k, 0, true, 1, false, 3});
+    }
+    add({false, k, 0, false, 1, false, 3});
+    if (!can_chain) {
+        add({true, 0, 0, false, 1, false, 3});
+        if (i + 1 < ks.size()) add({false, ks[i + 1], 0, false, 1, false, 3});
+        if (items(1) <= cus && max_ntr > 256) add({false, k, 256, false, 1, false, 3});
+        if (i > 0) add({false, ks[i - 1], 0, false, 1, false, 3});
+    }
+    return out;
+}
+
+/* One whole run from its start (the one-shot entry points): the decompositions
+ * are timed on iterations of the run itself, since none of them changes a
+ * result, so no iteration is run twice and nothing is saved and restored. A run
+ * of fewer than 6 launches takes the first candidate; others time one launch (8
+ * iterations where a launch holds one) of each candidate until a quarter of the
+ * run is spent. */
+void ggdmc_session::run_whole() {
+    uint32_t left = last_iter;
+    if (mode == GGDMC_FP64_PLAIN || d.S == 0 || decomp_given()) {
+        if (mode == GGDMC_FP64_PLAIN) {
+            run_plain(left);
+        } else {
+            capture((int)std::min<uint32_t>(64u, left));
+            run_batched(left);
+        }
+        return;
+    }
+    const std::vector<Decomp> cands = candidates();
+    size_t pick = 0;
+    while (!try_decomp(cands[pick])) ++pick;
+    auto run = [&](uint32_t cnt) {
+        run_batched(cnt);
+        left -= cnt;
+    };
+    auto unit = [&]() { return ipl > 1 ? (uint32_t)ipl : 8u; };
+    Event e0, e1;
+    auto timed = [&]() {
+        const uint32_t cnt = unit();
+        HIPCHECK(hipEventRecord(e0.get(), stream));
+        run(cnt);
+        HIPCHECK(hipEventRecord(e1.get(), stream));
+        HIPCHECK(hipEventSynchronize(e1.get()));
+        float ms = 0.f;
+        HIPCHECK(hipEventElapsedTime(&ms, e0.get(), e1.get()));
+        return ms / (float)cnt;
+    };
+    if (left >= 6 * unit()) {
+        const uint32_t total = left;
+        size_t now = pick;
+        run(unit());   /* the first launch of a process loads the code */
+        float best = timed();
+        for (size_t c = pick + 1; c < cands.size(); ++c) {
+            if (total - left > total / 4) break;
+            if (!try_decomp(cands[c])) continue;
+            now = c;
+            const float ms = timed();
+            if (ms < best) {
+                best = ms;
+                pick = c;
+            }
+        }
+        if (now != pick) try_decomp(cands[pick]);
+    }
+    /* one iteration per launch: replayed from a graph */
+    if (ipl == 1 && left >= 2) capture((int)std::min<uint32_t>(64u, left));
+    run(left);
+}
+
+/* The next n_iter iterations, or the whole run; waits for them, with their
+ * device time, trace and fault flag. */
+void ggdmc_session::run_timed(uint32_t n_iter, bool whole) {
+    if (d.trace) HIPCHECK(hipMemsetAsync(d.trace_n, 0, sizeof(uint32_t), stream));
+    HIPCHECK(hipEventRecord(ev0, stream));
+    if (whole) run_whole();
+    else if (mode == GGDMC_FP64_PLAIN) run_plain(n_iter);
+    else run_batched(n_iter);
+    HIPCHECK(hipEventRecord(ev1, stream));
+    HIPCHECK(hipEventSynchronize(ev1));
+    HIPCHECK(hipEventElapsedTime(&last_ms, ev0, ev1));
+    check_fault();
+    collect_trace();
+}
+
+/* Picks a session's work decomposition by timing graph replays of a few real
  * iterations of each candidate from a snapshot of the state, which is then
  * restored (results do not depend on the decomposition, only the time does). */
 void ggdmc_session::autotune() {
     if (d.S == 0) return;
-    struct Cand {
-        bool fused;
-        int k, tpt;
-        bool chained;
-        int ipl;
-        bool span;
-        int occ;
-    };
-    const int ngmax = (d.nchain + d.G - 1) / d.G;
-    std::vector<Cand> cands{{true, 0, 0, false, 1, false, 3}};
-    std::vector<int> ks;
-    for (int k : {1, 2, 4, 8, ngmax})
-        if (k <= ngmax && std::find(ks.begin(), ks.end(), k) == ks.end()) ks.push_back(k);
-    const bool can_chain = nsweep_sub == 1 && cfg.launch_mode != 1;
-    for (int one = 0; one < (can_chain ? 2 : 1); ++one)
-        for (int k : ks)
-            for (int t : {0, 256, 1024})
-                if (t == 0 || t < max_ntr) {
-                    const int64_t nt = t == 0 ? 1 : (max_ntr + t - 1) / t;
-                    if ((int64_t)d.S * ((ngmax + k - 1) / k) * nt <= ((int64_t)1 << 22)) {
-                        cands.push_back({false, k, t, one == 1, 1, false, 3});
-                        /* several iterations per launch: whole subjects, the
-                         * population step inside the launch; items of one
-                         * group, or spanning every group */
-                        if (one == 1 && t == 0 && cfg.launch_mode != 2) {
-                            /* the subject kernel at 3 and at 4 waves per SIMD */
-                            for (int oc : {3, 4}) {
-                                if (cfg.waves_per_simd != 0 && oc != cfg.waves_per_simd) continue;
-                                cands.push_back({false, k, t, true, kItersPerLaunch, false, oc});
-                                if (span_fits((ngmax + k - 1) / k))
-                                    cands.push_back({false, k, t, true, kItersPerLaunch, true, oc});
-                            }
-                        }
-                    }
-                }
+    const std::vector<Decomp> cands = candidates();
     const size_t nth = (size_t)d.S * d.nchain * d.P, nch = (size_t)d.S * d.nchain;
     const size_t nph = (size_t)d.n_phi * d.nchain * 2 * d.P, npc = (size_t)d.n_phi * d.nchain;
     const size_t nev = (size_t)std::max(d.S, 1);
@@ -987,17 +1175,12 @@ void ggdmc_session::autotune() {
     save();
     const uint32_t it0 = next_iter;
     float best = 1e30f;
-    Cand pick = cands[0];
+    Decomp pick = cands[0];
     /* iterations per timed replay: one launch of launch modes 3 and 4 when
      * the run has room for three (warm-up and two timed) */
     const int K = last_iter >= 3 * (uint32_t)kItersPerLaunch ? kItersPerLaunch : 16;
-    for (const Cand &c : cands) {
-        try {
-            set_decomp(c.fused, c.k, c.tpt, c.chained, c.ipl, c.span, c.occ);
-        } catch (const Error &) {
-            if (c.ipl == 1) throw;
-            continue;   /* no population step inside the launch for this design */
-        }
+    for (const Decomp &c : cands) {
+        if (!try_decomp(c)) continue;
         next_iter = it0;
         capture(K);
         run_batched(K); /* warm-up */
@@ -1105,9 +1288,7 @@ int ggdmc_session_create(const ggdmc_config *cfg, const ggdmc_model *model, cons
         s->build(cfg, model, jobs, njobs);
         if (s->mode != GGDMC_FP64_PLAIN) {
             /* tune the tile shape when the run is long enough to repay it */
-            if (cfg->trials_per_tile == 0 && cfg->chains_per_item == 0 && cfg->launch_mode < 2 &&
-                s->last_iter >= 64)
-                s->autotune();
+            if (!s->decomp_given() && s->last_iter >= 64) s->autotune();
             const uint32_t total = s->last_iter;
             const int K = (int)std::min<uint32_t>(64u, total);
             s->capture(K);
@@ -1128,16 +1309,8 @@ int ggdmc_session_advance(ggdmc_session *s, int32_t n_iter) {
     try {
         const uint32_t left = s->next_iter <= s->last_iter ? s->last_iter - s->next_iter + 1 : 0;
         const uint32_t n = std::min<uint32_t>((uint32_t)n_iter, left);
-        if (s->d.trace) HIPCHECK(hipMemsetAsync(s->d.trace_n, 0, sizeof(uint32_t), s->stream));
         if (s->mode != GGDMC_FP64_PLAIN) s->prepare_rest(n);
-        HIPCHECK(hipEventRecord(s->ev0, s->stream));
-        if (s->mode == GGDMC_FP64_PLAIN) s->run_plain(n);
-        else s->run_batched(n);
-        HIPCHECK(hipEventRecord(s->ev1, s->stream));
-        HIPCHECK(hipEventSynchronize(s->ev1));
-        HIPCHECK(hipEventElapsedTime(&s->last_ms, s->ev0, s->ev1));
-        s->check_fault();
-        s->collect_trace();
+        s->run_timed(n, false);
     } catch (const std::exception &e) {
         return fail(e);
     }
@@ -1199,9 +1372,8 @@ int ggdmc_session_profile(ggdmc_session *s, int32_t n_iter, double *subject_kern
         const uint32_t step = s->chained ? (uint32_t)s->ipl : 1u;
         for (uint32_t k = 0; k < n; k += step) {
             const int cnt = (int)std::min(step, n - k);
-            set_base_kernel<<<1, 1, 0, s->stream>>>(s->iter_base, s->next_iter);
-            HIPCHECK(hipGetLastError());
-            s->enqueue_iteration(0, &ev, cnt);
+            s->set_base(0);
+            s->enqueue_iteration(s->next_iter, &ev, cnt);
             s->next_iter += (uint32_t)cnt;
         }
         s->flush_store();
@@ -1280,16 +1452,23 @@ int ggdmc_last_trace(const ggdmc_trace_record **records, int64_t *n, int64_t *dr
 
 int ggdmc_run_batch(const ggdmc_config *cfg, const ggdmc_model *model, const ggdmc_job *jobs,
                     int32_t njobs) {
-    ggdmc_session *s = nullptr;
     g_trace.clear();
     g_trace_dropped = 0;
-    int rc = ggdmc_session_create(cfg, model, jobs, njobs, &s);
-    if (rc != GGDMC_OK) return rc;
-    rc = ggdmc_session_advance(s, (int32_t)s->last_iter);
-    if (rc == GGDMC_OK) rc = ggdmc_session_download(s);
+    if (ggdmc_device_count() < 1) {
+        g_error = "no gfx950 device visible";
+        return GGDMC_ENODEV;
+    }
+    auto s = std::make_unique<ggdmc_session>();
+    int rc = GGDMC_OK;
+    try {
+        s->build(cfg, model, jobs, njobs);
+        s->run_timed(0, true);
+    } catch (const std::exception &e) {
+        rc = fail(e);
+    }
+    if (rc == GGDMC_OK) rc = ggdmc_session_download(s.get());
     g_trace.swap(s->trace);
     g_trace_dropped = s->trace_dropped;
-    ggdmc_session_destroy(s);
     return rc;
 }
 

@@ -208,19 +208,18 @@ class JobSpec:
     nparameter_de: int = 0
 
 
-class Session:
-    """A batch of runs resident on the GPU (ggdmc_session_*)."""
+class _Batch:
+    """The C structures of a batch of runs and the buffers they point into."""
 
     def __init__(self, cfg, model, jobs):
-        L = _lib.lib()
         self.cfg = cfg
         self.keep = Keep()
         self.jobs = jobs
         k = self.keep
         P = model.npar if model is not None else jobs[0].p_prior.npar
         self.P = P
-        cm = model.c_struct(k) if model is not None else None
-        cjobs = (_lib.Job * len(jobs))()
+        self.cmodel = model.c_struct(k) if model is not None else None
+        cjobs = self.cjobs = (_lib.Job * len(jobs))()
         self.outs = []
         for i, j in enumerate(jobs):
             cj = cjobs[i]
@@ -263,10 +262,31 @@ class Session:
                     cj.nsubject = hd.shape[0]
                     cj.hyper_data = ptr(hd)
             self.outs.append(o)
-        k.items.extend([cm, cjobs])
+        k.items.extend([self.cmodel, cjobs])
+
+    def args(self):
+        return (C.byref(self.cfg), C.byref(self.cmodel) if self.cmodel is not None else None,
+                self.cjobs, len(self.jobs))
+
+    def results(self):
+        """Per job {'phi': Posterior|None, 'subjects': [Posterior]}."""
+        res = []
+        for j, o in zip(self.jobs, self.outs):
+            res.append({"phi": o["phi"].posterior(self.cfg, j.h_prior.pnames if j.h_prior else None)
+                        if o["phi"] is not None else None,
+                        "subjects": [x.posterior(self.cfg, j.p_prior.pnames) for x in o["subjects"]]})
+        return res
+
+
+class Session:
+    """A batch of runs resident on the GPU (ggdmc_session_*)."""
+
+    def __init__(self, cfg, model, jobs):
+        L = _lib.lib()
+        self.batch = _Batch(cfg, model, jobs)
+        self.cfg, self.jobs, self.P = cfg, jobs, self.batch.P
         h = C.c_void_p()
-        check(L.ggdmc_session_create(C.byref(cfg), C.byref(cm) if cm is not None else None,
-                                     cjobs, len(jobs), C.byref(h)))
+        check(L.ggdmc_session_create(*self.batch.args(), C.byref(h)))
         self.h = h
         self.total_iters = cfg.nmc * cfg.thin - 1
 
@@ -317,12 +337,7 @@ class Session:
     def download(self):
         """Returns per job {'phi': Posterior|None, 'subjects': [Posterior]}."""
         check(_lib.lib().ggdmc_session_download(self.h))
-        res = []
-        for j, o in zip(self.jobs, self.outs):
-            res.append({"phi": o["phi"].posterior(self.cfg, j.h_prior.pnames if j.h_prior else None)
-                        if o["phi"] is not None else None,
-                        "subjects": [x.posterior(self.cfg, j.p_prior.pnames) for x in o["subjects"]]})
-        return res
+        return self.batch.results()
 
     def close(self):
         if getattr(self, "h", None):
@@ -334,13 +349,20 @@ class Session:
 
 
 def run_batch(cfg, model, jobs):
-    """All jobs to completion in one session (ggdmc_run_batch)."""
-    s = Session(cfg, model, jobs)
-    try:
-        s.advance(s.total_iters)
-        return s.download()
-    finally:
-        s.close()
+    """All jobs to completion (ggdmc_run_batch)."""
+    b = _Batch(cfg, model, jobs)
+    check(_lib.lib().ggdmc_run_batch(*b.args()))
+    return b.results()
+
+
+def last_trace():
+    """Decision records of the last run_batch on this thread (pop_debug /
+    sub_debug), as Session.trace."""
+    p = C.POINTER(_lib.TraceRecord)()
+    n = C.c_int64()
+    dr = C.c_int64()
+    check(_lib.lib().ggdmc_last_trace(C.byref(p), C.byref(n), C.byref(dr)))
+    return _lib.trace_array(p, n.value), dr.value
 
 
 def run_subject(cfg, model, p_prior, data, start, seed):

@@ -20,7 +20,7 @@ import numpy as np
 
 from . import _lib
 from .priors import logdprior, rprior, sumloghlike, sumlogprior
-from .runs import JobSpec, PriorSpec, Posterior, Session, format_trace, loglike, make_config
+from .runs import JobSpec, PriorSpec, Posterior, format_trace, last_trace, loglike, make_config, run_batch
 
 
 def set_priors(p_prior, h_prior=None):
@@ -136,18 +136,14 @@ def _config(nmc, nchain, thin, kw):
 def _execute(kind, model, jobs, cfg):
     """Runs the jobs to completion; with a debug flag set, prints their
     decisions as the reference does (src/de.cpp:85-106)."""
-    s = Session(cfg, model, jobs)
-    try:
-        s.advance(s.total_iters)
-        if cfg.pop_debug or cfg.sub_debug:
-            rec, dropped = s.trace()
-            if len(rec):
-                print(format_trace(rec))
-            if dropped:
-                print("(%d further decisions not recorded)" % dropped)
-        return s.download()
-    finally:
-        s.close()
+    res = run_batch(cfg, model, jobs)
+    if cfg.pop_debug or cfg.sub_debug:
+        rec, dropped = last_trace()
+        if len(rec):
+            print(format_trace(rec))
+        if dropped:
+            print("(%d further decisions not recorded)" % dropped)
+    return res
 
 
 def StartSampling_subject(dmi, priors, samples_list=None, nmc=500, nchain=None, thin=1,

@@ -167,7 +167,9 @@ int ggdmc_run(const ggdmc_config *cfg, const ggdmc_model *model, const ggdmc_pri
               ggdmc_samples *phi_out, ggdmc_samples *subject_outs);
 
 /* Many independent runs (parallel_lapply's ncore runs, R/sampling.R:13-121;
- * recovery fits) in one launch sequence. All jobs share cfg and model. */
+ * recovery fits) in one launch sequence. All jobs share cfg and model. A work
+ * split left to the library is timed on the run's own iterations (it never
+ * changes results); a session times it when it is created. */
 int ggdmc_run_batch(const ggdmc_config *cfg, const ggdmc_model *model, const ggdmc_job *jobs,
                     int32_t njobs);
 
