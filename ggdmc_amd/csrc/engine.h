@@ -37,6 +37,7 @@ constexpr int kWaves = kBlock / 64;
 constexpr int kMaxChains = 256;    /* chains per run */
 constexpr int kChunk = 128;        /* trials per canonical chunk sum */
 constexpr int kStatBlock = 32;     /* subjects per block of the population statistics */
+constexpr uint32_t kHyperItersPerLaunch = 256; /* iterations per launch of hyper-only runs */
 constexpr int kItersPerLaunch = 32; /* iterations per subject launch in launch mode 3 */
 
 struct JobDev {

@@ -45,6 +45,8 @@ hipError_t ggdmc_internal_launch_sweep(const Dev *d, const SweepArgs *a, int mod
                                        hipStream_t stream);
 hipError_t ggdmc_internal_launch_phi(const Dev *d, uint32_t iter_off, size_t lds, int stats_lds,
                                      hipStream_t stream);
+hipError_t ggdmc_internal_launch_hyper(const Dev *d, uint32_t iter, int count, size_t lds, int stats_lds,
+                                       hipStream_t stream);
 hipError_t ggdmc_internal_launch_plain_subject(const Dev *d, uint32_t iter, int sweep, int j,
                                                hipStream_t stream);
 hipError_t ggdmc_internal_launch_plain_phi(const Dev *d, uint32_t iter, int sweep, int j,
@@ -825,7 +827,6 @@ void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chai
  * due. ev, if given, receives an event pair around every subject launch. */
 void ggdmc_session::enqueue_iteration(uint32_t off, std::vector<hipEvent_t> *ev, int count) {
     if (d.n_phi > 0 && !overlap) HIPCHECK(ggdmc_internal_launch_phi(&d, off, phi_lds, phi_stats_lds, stream));
-    if (d.S == 0) return;
     const int lk = mode == GGDMC_FP64_BATCHED ? GGDMC_FP64_BATCHED : GGDMC_MIXED_BATCHED;
     const int ngl = (fused || chained) ? 1 : d.G;
     for (int sw = 0; sw < nsweep_sub; ++sw) {
@@ -888,7 +889,7 @@ hipGraphExec_t ggdmc_session::make_graph(int K) {
 
 void ggdmc_session::capture(int K) {
     drop_graph();
-    if (K < 2) return;
+    if (K < 2 || d.S == 0) return;
     graph = make_graph(K);
     graph_iters = K;
 }
@@ -922,7 +923,10 @@ void ggdmc_session::run_batched(uint32_t n_iter) {
     if (n_iter == 0) return;
     while (n_iter > 0) {
         uint32_t cnt;
-        if (graph && n_iter >= (uint32_t)graph_iters) {
+        if (d.S == 0) {
+            cnt = std::min<uint32_t>(n_iter, kHyperItersPerLaunch);
+            HIPCHECK(ggdmc_internal_launch_hyper(&d, next_iter, (int)cnt, phi_lds, phi_stats_lds, stream));
+        } else if (graph && n_iter >= (uint32_t)graph_iters) {
             set_base(next_iter);
             HIPCHECK(hipGraphLaunch(graph, stream));
             cnt = (uint32_t)graph_iters;
