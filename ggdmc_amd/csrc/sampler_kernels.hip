@@ -319,13 +319,6 @@ __device__ __forceinline__ double subject_prior_term_cached(const Dev &d, const 
     return __builtin_nan("");
 }
 
-/* sumlogprior (src/de.cpp:144, :186) of x: terms added in parameter order. */
-__device__ double subject_logprior(const Dev &d, const JobDev &job, int chain, const double *x) {
-    double s = 0.0;
-    for (int p = 0; p < d.P; ++p) s += subject_prior_term(d, job, chain, p, x[p]);
-    return s;
-}
-
 __device__ __forceinline__ bool mh_accept(double tpost, double cur, double U) {
     const double ratio = exp_acc(tpost - cur, g_exp2tab);
     if (ratio != ratio) return false;
@@ -940,13 +933,6 @@ __device__ __forceinline__ double hyper_prior_term_cached(const PhiLds &L, int q
 }
 
 
-
-/* sumlogprior of a population state x (src/de.cpp:426, :518): 2P terms in order. */
-__device__ double hyper_logprior(const Dev &d, const JobDev &job, const double *x) {
-    double s = 0.0;
-    for (int q = 0; q < 2 * d.P; ++q) s += hyper_prior_term(d, job, q, x[q]);
-    return s;
-}
 
 /* Sufficient statistics (mean, M2, min, max) of the run's S subject values
  * of every (chain, parameter) pair q = chain * P + parameter, in a fixed
@@ -2072,17 +2058,18 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
 /* ------------------------------------------------------- plain FP64 path */
 /* Step j of the sequential sweep of every subject: crossover of chain j, or
  * migration ring step j (src/de.cpp:567-665, :111-199), reference arithmetic.
- * One workgroup per subject over all its trials. */
+ * One workgroup per subject over all its trials; one thread per parameter
+ * makes the proposal and its prior term (one thread for all of them, with a
+ * Philox block and a logarithm or two each in a row, cost a fifth of a step: 18
+ * chains, 6 parameters, 768 trials 14.7 us a step, launch gap included, now
+ * 11.7), summed in parameter order. */
 __global__ __launch_bounds__(kBlock) void plain_subject_kernel(Dev d, uint32_t iter, int sweep, int j) {
-    __shared__ double prop[64];
+    __shared__ double prop[64], term[64];
     __shared__ double red[kWaves];
     __shared__ AccK acck[256];
     __shared__ int sub[kMaxChains];
-    __shared__ int info[4];
-    __shared__ double misc[2];
+    __shared__ int info[2];
     const int s = blockIdx.x;
-    stage_tables(d);
-    __syncthreads();   /* thread 0 takes the prior terms before the next barrier */
     const JobDev job = d.jobs[d.subj_job[s]];
     const int n = d.nchain, P = d.P;
     const bool single = job.kind != GGDMC_KIND_HIER;
@@ -2092,48 +2079,42 @@ __global__ __launch_bounds__(kBlock) void plain_subject_kernel(Dev d, uint32_t i
     const int dsweep = (blocked && single) ? 0 : sweep;
     const Stream sd = make_stream(seed, iter + d.philox_offset, (uint32_t)d.subj_unit[s], (uint32_t)dsweep);
     const bool migrate = decision_u(sd) < d.sub_mig;
-    double *th = d.theta + (size_t)s * n * P;
-    if (threadIdx.x == 0) {
-        info[0] = 0; /* active */
-        if (migrate) {
+    /* crossover: chain j from partners m0, m1; migration: S_j into S_{j+1} */
+    int src = j, dst = j, m0 = j, m1 = j;
+    double U = 0.0;
+    Stream st = sd;
+    if (migrate) {
+        if (threadIdx.x == 0) {
             const bool act = blocked && single ? sweep == 0 : true;
             const int ns = act ? subchains(sd, n, sub) : 0;
-            if (j < ns) {
-                const int src = sub[j], dst = sub[(j + 1) % ns];
-                const int para = (blocked && !single) ? sweep : -1;
-                const uint32_t slot = kSlotMigrate | (uint32_t)j;
-                for (int p = 0; p < P; ++p) prop[p] = th[src * P + p];
-                if (para >= 0) prop[para] += jitter(sd, slot, 0, d.rp);
-                else
-                    for (int p = 0; p < P; ++p) prop[p] += jitter(sd, slot, p, d.rp);
-                const U4 b = sd.block(slot, 0);
-                misc[0] = u53(b.x[0], b.x[1]);
-                misc[1] = subject_logprior(d, job, src, prop);
-                info[0] = 1;
-                info[1] = dst;
-                info[2] = src;
-            }
-        } else {
-            const int para = blocked ? sweep : -1;
-            const Stream st = make_stream(seed, iter + d.philox_offset, (uint32_t)d.subj_unit[s], (uint32_t)sweep);
-            int m0, m1;
-            double U;
-            partners(st, j, j, j + 1, n, m0, m1, U);
-            for (int p = 0; p < P; ++p) prop[p] = th[j * P + p];
-            if (para >= 0) {
-                prop[para] += jitter(st, (uint32_t)j, 0, d.rp) + job.gamma * (th[m0 * P + para] - th[m1 * P + para]);
-            } else {
-                for (int p = 0; p < P; ++p)
-                    prop[p] += jitter(st, (uint32_t)j, p, d.rp) + job.gamma * (th[m0 * P + p] - th[m1 * P + p]);
-            }
-            misc[0] = U;
-            misc[1] = subject_logprior(d, job, j, prop);
-            info[0] = 1;
-            info[1] = j;
+            info[0] = j < ns ? sub[j] : -1;
+            info[1] = j < ns ? sub[(j + 1) % ns] : -1;
         }
+        __syncthreads();
+        src = info[0];
+        dst = info[1];
+        if (src < 0) return;
+        const U4 b = sd.block(kSlotMigrate | (uint32_t)j, 0);
+        U = u53(b.x[0], b.x[1]);
+    } else {
+        st = make_stream(seed, iter + d.philox_offset, (uint32_t)d.subj_unit[s], (uint32_t)sweep);
+        partners(st, j, j, j + 1, n, m0, m1, U);
+    }
+    stage_tables(d);
+    __syncthreads();
+    double *th = d.theta + (size_t)s * n * P;
+    const int para = migrate ? (blocked && !single ? sweep : -1) : (blocked ? sweep : -1);
+    const uint32_t slot = migrate ? kSlotMigrate | (uint32_t)j : (uint32_t)j;
+    for (int p = threadIdx.x; p < P; p += blockDim.x) {
+        double x = th[src * P + p];
+        if (para < 0 || p == para) {
+            const double jit = jitter(st, slot, para < 0 ? (uint32_t)p : 0u, d.rp);
+            x += migrate ? jit : jit + job.gamma * (th[m0 * P + p] - th[m1 * P + p]);
+        }
+        prop[p] = x;
+        term[p] = subject_prior_term(d, job, src, p, x);
     }
     __syncthreads();
-    if (!info[0]) return;
     for (int e = threadIdx.x; e < d.n_cond * d.n_acc; e += blockDim.x)
         make_acck<DevOps>(prop, d.par_src + e * 6, d.par_const + e * 6, acck[e]);
     __syncthreads();
@@ -2145,25 +2126,24 @@ __global__ __launch_bounds__(kBlock) void plain_subject_kernel(Dev d, uint32_t i
     }
     const double tll = block_sum(acc, red);
     if (threadIdx.x == 0) {
-        const int dst = info[1];
+        double tlp = 0.0;
+        for (int p = 0; p < P; ++p) tlp += term[p];
         atomicAdd(d.evals + s, (unsigned long long)(t_hi - t_lo));
         const double cur = d.lp[(size_t)s * n + dst] + d.ll[(size_t)s * n + dst];
-        const bool acc = mh_accept(misc[1] + tll, cur, misc[0]);
-        if (__builtin_expect(subject_traced(d, s), 0)) {
-            /* crossover records carry the sweep of their stream, migration
-             * steps the decision's */
-            const Stream tr = migrate ? sd
-                                      : make_stream(seed, iter + d.philox_offset, (uint32_t)d.subj_unit[s],
-                                                    (uint32_t)sweep);
-            trace_put(d, d.subj_job[s], d.subj_unit[s], tr, migrate ? 1 : 0, j, migrate ? info[2] : j, dst,
-                      misc[1], tll, cur, acc);
-        }
+        const bool acc = mh_accept(tlp + tll, cur, U);
+        /* crossover records carry the sweep of their stream, migration steps
+         * the decision's */
+        if (__builtin_expect(subject_traced(d, s), 0))
+            trace_put(d, d.subj_job[s], d.subj_unit[s], st, migrate ? 1 : 0, j, src, dst, tlp, tll, cur, acc);
+        info[0] = acc;
         if (acc) {
-            for (int p = 0; p < P; ++p) th[dst * P + p] = prop[p];
-            d.lp[(size_t)s * n + dst] = misc[1];
+            d.lp[(size_t)s * n + dst] = tlp;
             d.ll[(size_t)s * n + dst] = tll;
         }
     }
+    __syncthreads();
+    if (info[0])
+        for (int p = threadIdx.x; p < P; p += blockDim.x) th[dst * P + p] = prop[p];
 }
 
 /* Naive sumloghlike over subject states of chain c (src/de.cpp:245-270). */
@@ -2187,11 +2167,10 @@ __device__ double plain_hyper_ll(const Dev &d, const JobDev &job, const double *
 __global__ __launch_bounds__(kBlock) void plain_phi_kernel(Dev d, uint32_t iter, int sweep, int j,
                                                           const double *hyper_rows,
                                                           const int64_t *hyper_off) {
-    __shared__ double prop[128];
+    __shared__ double prop[128], term[128];
     __shared__ double red[kWaves];
     __shared__ int sub[kMaxChains];
     __shared__ int info[4];
-    __shared__ double misc[4];
     const int f = blockIdx.x;
     stage_tables(d);
     const JobDev job = d.jobs[d.phi_job[f]];
@@ -2237,50 +2216,46 @@ __global__ __launch_bounds__(kBlock) void plain_phi_kernel(Dev d, uint32_t iter,
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        const int para = blocked && (hier || info[0] == 1) ? sweep : -1;
-        if (info[0] == 2) {
-            const uint32_t slot = kSlotMigrate | (uint32_t)j;
-            for (int p = 0; p < P2; ++p) prop[p] = ph[(size_t)src * P2 + p];
-            const int mp = (blocked && hier) ? sweep : -1;
-            if (mp >= 0) prop[mp] += jitter(sd, slot, 0, d.rp);
-            else
-                for (int p = 0; p < P2; ++p) prop[p] += jitter(sd, slot, p, d.rp);
-            const U4 b = sd.block(slot, 0);
-            misc[0] = u53(b.x[0], b.x[1]);
-        } else {
-            const Stream st = make_stream(seed, iter + d.philox_offset, unit, (uint32_t)sweep);
-            int m0, m1;
-            double U;
-            partners(st, j, j, j + 1, n, m0, m1, U);
-            for (int p = 0; p < P2; ++p) prop[p] = ph[(size_t)j * P2 + p];
-            if (para >= 0) {
-                prop[para] += jitter(st, (uint32_t)j, 0, d.rp) +
-                              job.gamma * (ph[(size_t)m0 * P2 + para] - ph[(size_t)m1 * P2 + para]);
-            } else {
-                for (int p = 0; p < P2; ++p)
-                    prop[p] += jitter(st, (uint32_t)j, p, d.rp) +
-                               job.gamma * (ph[(size_t)m0 * P2 + p] - ph[(size_t)m1 * P2 + p]);
-            }
-            misc[0] = U;
+    /* the proposal and its prior terms, one thread per parameter */
+    const Stream st = info[0] == 2 ? sd : make_stream(seed, iter + d.philox_offset, unit, (uint32_t)sweep);
+    const bool ring = info[0] == 2;
+    const int para = ring ? (blocked && hier ? sweep : -1) : (blocked ? sweep : -1);
+    const uint32_t slot = ring ? kSlotMigrate | (uint32_t)j : (uint32_t)j;
+    int m0 = j, m1 = j;
+    double U;
+    if (ring) {
+        const U4 b = sd.block(slot, 0);
+        U = u53(b.x[0], b.x[1]);
+    } else {
+        partners(st, j, j, j + 1, n, m0, m1, U);
+    }
+    for (int q = threadIdx.x; q < P2; q += blockDim.x) {
+        double x = ph[(size_t)src * P2 + q];
+        if (para < 0 || q == para) {
+            const double jit = jitter(st, slot, para < 0 ? (uint32_t)q : 0u, d.rp);
+            x += ring ? jit : jit + job.gamma * (ph[(size_t)m0 * P2 + q] - ph[(size_t)m1 * P2 + q]);
         }
-        misc[1] = hyper_logprior(d, job, prop);
+        prop[q] = x;
+        term[q] = hyper_prior_term(d, job, q, x);
     }
     __syncthreads();
     const double tll = plain_hyper_ll(d, job, prop, src, rows, red);
     if (threadIdx.x == 0) {
+        double tlp = 0.0;
+        for (int q = 0; q < P2; ++q) tlp += term[q];
         const double cur = plp[dst] + pll[dst];
-        const bool acc = mh_accept(misc[1] + tll, cur, misc[0]);
-        if (__builtin_expect(phi_traced(d, job), 0)) {
-            const Stream tr = info[0] == 2 ? sd : make_stream(seed, iter + d.philox_offset, unit, (uint32_t)sweep);
-            trace_put(d, d.phi_job[f], -1, tr, info[0] == 2 ? 1 : 0, j, src, dst, misc[1], tll, cur, acc);
-        }
+        const bool acc = mh_accept(tlp + tll, cur, U);
+        if (__builtin_expect(phi_traced(d, job), 0))
+            trace_put(d, d.phi_job[f], -1, st, ring ? 1 : 0, j, src, dst, tlp, tll, cur, acc);
+        info[3] = acc;
         if (acc) {
-            for (int p = 0; p < P2; ++p) ph[(size_t)dst * P2 + p] = prop[p];
-            plp[dst] = misc[1];
+            plp[dst] = tlp;
             pll[dst] = tll;
         }
     }
+    __syncthreads();
+    if (info[3])
+        for (int q = threadIdx.x; q < P2; q += blockDim.x) ph[(size_t)dst * P2 + q] = prop[q];
 }
 
 /* Thinned store of every subject and (unless subjects_only) population
