@@ -40,6 +40,19 @@ constexpr int kStatBlock = 32;     /* subjects per block of the population stati
 constexpr uint32_t kHyperItersPerLaunch = 256; /* iterations per launch of hyper-only runs */
 constexpr int kItersPerLaunch = 32; /* iterations per subject launch in launch mode 3 */
 
+/* Division of 0 <= x <= 2^16 by a number d < 2^14 fixed for a launch:
+ * floor(x / d) = high word of (2x + 1) ceil(2^31 / d), as (2x + 1) / (2d) is at
+ * least 1 / (2d) below the next integer and the rounded multiplier adds less
+ * than 2^-15 (checked for every x and d <= 512). A division by a run-time value
+ * takes about 30 dependent instructions. */
+struct FastDiv {
+    uint32_t m;
+    uint32_t d;
+};
+inline FastDiv fast_div(int d) {
+    return FastDiv{(uint32_t)(((uint64_t(1) << 31) + (uint64_t)d - 1) / (uint64_t)d), (uint32_t)d};
+}
+
 struct JobDev {
     int32_t kind;           /* GGDMC_KIND_* */
     uint32_t k0, k1;        /* Philox key */
@@ -53,6 +66,11 @@ struct JobDev {
 struct Dev {
     int32_t P, n_acc, n_cond, nchain, G, nmc, thin;
     int32_t blocked_sub, blocked_pop;
+    FastDiv by_P, by_2P;        /* quotients by P, 2P */
+    FastDiv by_pb, by_2pb;      /* by the Philox blocks of P, 2P jitters */
+    FastDiv by_per;             /* by n_cond * n_acc */
+    FastDiv by_G;
+    uint64_t thin_m;            /* floor(2^64 / thin) + 1, 0 for thin 1 */
     double rp, sub_mig, pop_mig;
     int32_t S, n_phi, n_jobs;
     int32_t tpt;                /* trials per tile of trial-split items (multiple of kChunk) */
@@ -135,6 +153,7 @@ struct SweepArgs {
     int32_t chained;      /* every chain group in this launch: items carry their group, an
                              item waits for the previous group's items of its subject */
     int32_t rmax;         /* chain ranges per group (item_ready stride) */
+    FastDiv by_k, by_r;   /* quotients by kmax, rmax */
     int32_t tiles;        /* some subject's trials are split over several items */
     int32_t iters;        /* consecutive iterations in this launch (chained only; else 1): the
                              grid is iters segments of seg_wgs workgroups, segment s running

@@ -499,6 +499,13 @@ void ggdmc_session::build(const ggdmc_config *c, const ggdmc_model *model, const
     d.n_phi = F;
     d.n_jobs = nj;
     d.philox_offset = (uint32_t)cfg.iter_offset;
+    d.by_P = fast_div(P);
+    d.by_2P = fast_div(2 * P);
+    d.by_pb = fast_div((P + 3) / 4);
+    d.by_2pb = fast_div((2 * P + 3) / 4);
+    d.by_per = fast_div(d.n_cond * d.n_acc);
+    d.by_G = fast_div(G);
+    d.thin_m = cfg.thin == 1 ? 0 : ~uint64_t(0) / (uint64_t)cfg.thin + 1;
 
     if (any_lba) {
         d.par_src = pool.upload(cond.src, stream);
@@ -843,7 +850,7 @@ void ggdmc_session::enqueue_iteration(uint32_t off, std::vector<hipEvent_t> *ev,
             const int seg_wgs = multi > 1 ? (pw + list_n[g] + 7) / 8 * 8 : pw + list_n[g];
             SweepArgs a{off, sw, (fused || chained) ? 0 : g, (fused || chained) ? d.G : g + 1, (int)store,
                         chain_batch, kmax, cmax, tstage, list_n[g], lists[g],
-                        pw, ovl_stats_lds, (int)chained, rmax, (int)tiled, multi, seg_wgs, (int)span};
+                        pw, ovl_stats_lds, (int)chained, rmax, fast_div(kmax), fast_div(rmax), (int)tiled, multi, seg_wgs, (int)span};
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (ev) {
                 HIPCHECK(hipEventCreate(&e0));
@@ -1666,6 +1673,7 @@ static int loglike_impl(const ggdmc_model *model, const ggdmc_subject *data, con
         d.P = P;
         d.n_acc = na;
         d.n_cond = nq;
+        d.by_per = fast_div(nq * na);
         d.nchain = 1;
         d.par_src = reinterpret_cast<const int32_t *>(b + o_src);
         d.par_const = reinterpret_cast<const double *>(b + o_const);

@@ -113,9 +113,6 @@ GGDMC_RFN double decision_u(const Stream &st) {
     return u53(b.x[0], b.x[1]);
 }
 
-/* Chain groups of a sweep: group g = chains [g*n/G, (g+1)*n/G). */
-GGDMC_RFN int group_lo(int g, int n, int G) { return (g * n) / G; }
-
 /* Two distinct partners of chain i drawn from the chains outside [lo, hi),
  * plus the accept U (src/de.cpp:54-60 draws a random ordered pair from the
  * chains other than i; with one chain per group this is the same law). */

@@ -66,6 +66,23 @@ struct DevOps {
     static __device__ __forceinline__ double log(double x) { return log_acc(x); }
 };
 
+__device__ __forceinline__ int quo(int x, FastDiv f) { return (int)__umulhi(2u * (uint32_t)x + 1u, f.m); }
+
+/* Chain groups of a sweep: group g = chains [g*n/G, (g+1)*n/G); its first
+ * chain, its size, and its chain ranges. */
+__device__ __forceinline__ int glo(const Dev &d, int g) { return quo(g * d.nchain, d.by_G); }
+__device__ __forceinline__ int gsize(const Dev &d, int g) { return glo(d, g + 1) - glo(d, g); }
+__device__ __forceinline__ int ranges(const Dev &d, const SweepArgs &a, int g) {
+    return quo(gsize(d, g) + a.kmax - 1, a.by_k);
+}
+
+/* Whether iteration iter is stored, and its column. */
+__device__ __forceinline__ bool stored(const Dev &d, uint32_t iter, int &col) {
+    const uint32_t q = d.thin_m == 0 ? iter : (uint32_t)__umul64hi((uint64_t)iter, d.thin_m);
+    col = (int)q;
+    return q * (uint32_t)d.thin == iter && col < d.nmc;
+}
+
 enum { MODE_MIXED = 0, MODE_NAIVE = 1 };
 
 constexpr int kAccKDoubles = sizeof(AccK) / sizeof(double);
@@ -209,7 +226,8 @@ __device__ __forceinline__ void chunk_sums(const Dev &d, const TrialView &tv, in
                                            uint32_t *pend) {
     static_assert(kChunk == 128, "two trials per lane");
     const int lane = threadIdx.x & 63;
-    /* the wave index is uniform: keep the unit loop scalar */
+    /* the wave index is uniform: keep the unit loop scalar, without a division
+     * per unit */
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
     const int per_chain = d.n_cond * d.n_acc;
     const int nu = kb * nj;
@@ -217,8 +235,13 @@ __device__ __forceinline__ void chunk_sums(const Dev &d, const TrialView &tv, in
         for (int w = threadIdx.x; w < (nu + 31) / 32; w += blockDim.x) pend[w] = 0u;
         __syncthreads();
     }
-    for (int u = wave; u < nu; u += nw) {
-        const int c = u / nj, jj = u - c * nj;
+    /* unit u = (chain c, chunk jj); waves step by nw units */
+    int c = 0, jj = wave;
+    for (int u = wave; u < nu; u += nw, jj += nw) {
+        while (jj >= nj) {
+            jj -= nj;
+            ++c;
+        }
         double v = 0.0;
         if (active[c]) {
             const AccK *kc = reinterpret_cast<const AccK *>(acck) + (size_t)c * per_chain;
@@ -484,7 +507,7 @@ __device__ __forceinline__ void build_acck(const Dev &d, const SweepLds &L, cons
     const int per_chain = d.n_cond * d.n_acc;
     AccK *K = reinterpret_cast<AccK *>(acck);
     for (int e = threadIdx.x; e < kb * per_chain; e += blockDim.x) {
-        const int c = e / per_chain, r = e - c * per_chain;
+        const int c = quo(e, d.by_per), r = e - c * per_chain;
         make_acck<DevOps>(prop + (size_t)(cb + c) * P, L.psrc + r * 6, L.pcst + r * 6, K[e]);
     }
 }
@@ -494,7 +517,7 @@ __device__ __forceinline__ void build_acck(const Dev &d, const SweepLds &L, cons
 __device__ __forceinline__ void proposal_priors(const Dev &d, const JobDev &job, const SweepLds &L, int i0, int k) {
     const int P = d.P;
     for (int e = threadIdx.x; e < k * P; e += blockDim.x) {
-        const int c = e / P, p = e - c * P;
+        const int c = quo(e, d.by_P), p = e - c * P;
         L.tm[e] = subject_prior_term_cached(d, job, i0 + c, p, L.prop[e]);
     }
     __syncthreads();
@@ -521,7 +544,7 @@ __device__ __forceinline__ void proposal_stage1(const Dev &d, const JobDev &job,
     const int P = d.P, n = d.nchain;
     const int nb = para >= 0 ? 1 : (P + 3) >> 2;
     for (int e = threadIdx.x; e < k * nb; e += blockDim.x) {
-        const int c = e / nb, b = e - c * nb;
+        const int c = para >= 0 ? e : quo(e, d.by_pb), b = e - c * nb;
         const int i = i0 + c;
         if (b == 0) {
             int m0, m1;
@@ -546,7 +569,7 @@ __device__ __forceinline__ void proposal_stage1(const Dev &d, const JobDev &job,
     /* late: the population step is still running, the priors come after the
      * likelihoods (late_prior) */
     for (int e = threadIdx.x; e < (late ? 0 : k * P); e += blockDim.x) {
-        const int c = e / P, p = e - c * P;
+        const int c = quo(e, d.by_P), p = e - c * P;
         double *q = L.pri + (size_t)e * 4;
         if (hier) {
             const size_t r = ((size_t)job.phi_index * n + i0 + c) * P + p;
@@ -588,7 +611,7 @@ __device__ __forceinline__ void proposal_stage2(const Dev &d, const JobDev &job,
                                 int para, bool late) {
     const int P = d.P;
     for (int e = threadIdx.x; e < k * P; e += blockDim.x) {
-        const int c = e / P, p = e - c * P;
+        const int c = quo(e, d.by_P), p = e - c * P;
         const double xi = L.th[(size_t)(i0 + c) * P + p];
         double x = xi;
         if (para < 0 || p == para)
@@ -681,7 +704,7 @@ __device__ __forceinline__ void accept_proposals(const Dev &d, const SweepLds &L
      * several iterations per launch, a later iteration's) may read the rows
      * in the same launch */
     for (int e = threadIdx.x; e < k * P; e += blockDim.x) {
-        const int c = e / P;
+        const int c = quo(e, d.by_P);
         if (!L.acc[c]) continue;
         const size_t r = (size_t)(i0 + c) * P + (e - c * P);
         L.th[r] = L.prop[e];
@@ -756,9 +779,8 @@ __device__ __forceinline__ void subject_migration(const Dev &d, const SweepLds &
  * subject's rows, in LDS). */
 __device__ __forceinline__ void store_chains(const Dev &d, const double *th, const double *lp, const double *ll,
                                              int x, uint32_t iter, int i0, int k) {
-    if (iter % (uint32_t)d.thin != 0) return;
-    const int col = (int)(iter / (uint32_t)d.thin);
-    if (col >= d.nmc || k <= 0) return;
+    int col;
+    if (!stored(d, iter, col) || k <= 0) return;
     const int n = d.nchain, P = d.P;
     double *ot = d.out_theta + ((size_t)x * d.nmc + col) * n * P;
     for (int e = threadIdx.x; e < k * P; e += blockDim.x) ot[(size_t)i0 * P + e] = th[(size_t)i0 * P + e];
@@ -1133,7 +1155,7 @@ __device__ __forceinline__ void phi_crossover(const Dev &d, const JobDev &job, c
     /* partners, accept U and jitter: one thread per (chain, Philox block) */
     const int nb = para >= 0 ? 1 : (P2 + 3) >> 2;
     for (int e = threadIdx.x; e < ng * nb; e += blockDim.x) {
-        const int c = e / nb, b = e - c * nb;
+        const int c = para >= 0 ? e : quo(e, d.by_2pb), b = e - c * nb;
         const int i = lo + c;
         int m0, m1;
         double U;
@@ -1159,11 +1181,11 @@ __device__ __forceinline__ void phi_crossover(const Dev &d, const JobDev &job, c
      * [3P, 4P) refreshed current shares (src/de.cpp:397); one loop per kind so
      * that a wave runs one kind of term */
     for (int e = threadIdx.x; e < ng * P2; e += blockDim.x) {
-        const int c = e / P2, q = e - c * P2;
+        const int c = quo(e, d.by_2P), q = e - c * P2;
         L.tm[(size_t)c * 4 * P + q] = hyper_prior_term_cached(L, q, L.prop[e]);
     }
     for (int e = threadIdx.x; e < ng * P; e += blockDim.x) {
-        const int c = e / P, p = e - c * P;
+        const int c = quo(e, d.by_P), p = e - c * P;
         const int i = lo + c;
         const double *x = L.prop + (size_t)c * P2;
         double *lc = L.pp + (size_t)e * 2;
@@ -1173,7 +1195,7 @@ __device__ __forceinline__ void phi_crossover(const Dev &d, const JobDev &job, c
     }
     if (hier) {
         for (int e = threadIdx.x; e < ng * P; e += blockDim.x) {
-            const int c = e / P, p = e - c * P;
+            const int c = quo(e, d.by_P), p = e - c * P;
             const int i = lo + c;
             const double *cur = L.ph + (size_t)i * P2;
             L.tm[(size_t)c * 4 * P + 3 * P + p] = hll_term(L, p, cur[p], cur[P + p],
@@ -1206,7 +1228,7 @@ __device__ __forceinline__ void phi_crossover(const Dev &d, const JobDev &job, c
     }
     __syncthreads();
     for (int e = threadIdx.x; e < ng * P2; e += blockDim.x) {
-        const int c = e / P2;
+        const int c = quo(e, d.by_2P);
         if (L.acc[c]) {
             L.ph[(size_t)lo * P2 + e] = L.prop[e];
             L.pc[(size_t)lo * P * 2 + e] = L.pp[e];   /* P2 == 2P entries per chain */
@@ -1220,7 +1242,7 @@ __device__ __forceinline__ void phi_crossover(const Dev &d, const JobDev &job, c
 __device__ __forceinline__ void phi_fill_consts(const Dev &d, const PhiLds &L) {
     const int P = d.P, P2 = 2 * P;
     for (int e = threadIdx.x; e < d.nchain * P; e += blockDim.x) {
-        const int c = e / P, p = e - c * P;
+        const int c = quo(e, d.by_P), p = e - c * P;
         if (L.sub[c] == 0)
             phi_log_consts(L, p, L.ph[(size_t)c * P2 + p], L.ph[(size_t)c * P2 + P + p], L.pc + (size_t)e * 2);
     }
@@ -1231,7 +1253,7 @@ __device__ __forceinline__ void phi_fill_consts(const Dev &d, const PhiLds &L) {
  * (src/de.cpp:272-383) on the state in LDS. */
 __device__ __forceinline__ void phi_sweeps(const Dev &d, const JobDev &job, uint32_t iter, const PhiLds &L,
                                            const double *stats) {
-    const int n = d.nchain, P2 = 2 * d.P, G = d.G;
+    const int P2 = 2 * d.P, G = d.G;
     const bool hier = job.kind == GGDMC_KIND_HIER;
     const uint32_t unit = hier ? kUnitPhi : 0u;
     const double mig = hier ? d.pop_mig : d.sub_mig;
@@ -1250,7 +1272,7 @@ __device__ __forceinline__ void phi_sweeps(const Dev &d, const JobDev &job, uint
         }
         const Stream st = make_stream(seed, iter + d.philox_offset, unit, (uint32_t)sw);
         for (int g = 0; g < G; ++g)
-            phi_crossover(d, job, L, st, group_lo(g, n, G), group_lo(g + 1, n, G), blocked ? sw : -1,
+            phi_crossover(d, job, L, st, glo(d, g), glo(d, g + 1), blocked ? sw : -1,
                           stats, hier);
     }
 }
@@ -1258,9 +1280,8 @@ __device__ __forceinline__ void phi_sweeps(const Dev &d, const JobDev &job, uint
 /* Thinned store of state f after iteration iter, from LDS. */
 __device__ __forceinline__ void phi_store(const Dev &d, int f, uint32_t iter, const PhiLds &L) {
     const int n = d.nchain, P2 = 2 * d.P;
-    if (iter % (uint32_t)d.thin != 0) return;
-    const int k = (int)(iter / (uint32_t)d.thin);
-    if (k >= d.nmc) return;
+    int k;
+    if (!stored(d, iter, k)) return;
     double *ot = d.phi_out_theta + ((size_t)f * d.nmc + k) * n * P2;
     for (int e = threadIdx.x; e < n * P2; e += blockDim.x) ot[e] = L.ph[e];
     for (int c = threadIdx.x; c < n; c += blockDim.x) {
@@ -1425,17 +1446,17 @@ __device__ __forceinline__ void wait_chains(const Dev &d, int f, int c_lo, int c
 template <bool AG>
 __device__ __forceinline__ void phi_chain(const Dev &d, int f, int i, uint32_t iter, char *lds_raw,
                                           bool chained) {
-    const int n = d.nchain, P = d.P, P2 = 2 * P, G = d.G;
+    const int n = d.nchain, P = d.P, P2 = 2 * P;
     const JobDev job = d.phi_jobs[f];
     const int S = job.nsubject, nblk = (S + kStatBlock - 1) / kStatBlock;
     const int t = threadIdx.x, bs = blockDim.x;
     int g = 0;
-    while (group_lo(g + 1, n, G) <= i) ++g;
+    while (glo(d, g + 1) <= i) ++g;
     const uint64_t seed = ((uint64_t)job.k1 << 32) | job.k0;
     const Stream st = make_stream(seed, iter + d.philox_offset, kUnitPhi, 0u);
     int m0, m1;
     double U;
-    partners(st, i, group_lo(g, n, G), group_lo(g + 1, n, G), n, m0, m1, U);
+    partners(st, i, glo(d, g), glo(d, g + 1), n, m0, m1, U);
 
     PhiLds L{};   /* the term helpers read hc, hd, sb */
     double *p = reinterpret_cast<double *>(lds_raw);
@@ -1543,7 +1564,7 @@ __device__ __forceinline__ void phi_chain(const Dev &d, int f, int i, uint32_t i
      * chains after their step of this iteration (device-scope loads; the
      * statistics above did not need them), and the later groups' chains wait
      * for this one before they change theirs. */
-    if (chained && g > 0) wait_chains(d, f, 0, group_lo(g, n, G), iter, false);
+    if (chained && g > 0) wait_chains(d, f, 0, glo(d, g), iter, false);
     {
         const double *r0 = d.phi + (off + m0) * P2, *r1 = d.phi + (off + m1) * P2;
         for (int r = t; r < P2; r += bs) {
@@ -1592,8 +1613,9 @@ __device__ __forceinline__ void phi_chain(const Dev &d, int f, int i, uint32_t i
     }
     __syncthreads();
     const bool acc = flag[1] != 0;
-    const bool out = iter % (uint32_t)d.thin == 0 && (int)(iter / (uint32_t)d.thin) < d.nmc;
-    const size_t ko = out ? (size_t)f * d.nmc + iter / (uint32_t)d.thin : 0;
+    int col;
+    const bool out = stored(d, iter, col);
+    const size_t ko = out ? (size_t)f * d.nmc + col : 0;
     for (int e = t; e < P2; e += bs) {
         const double x = acc ? prop[e] : xi[e];
         d.phi[(off + i) * P2 + e] = x;
@@ -1691,12 +1713,11 @@ __device__ __forceinline__ void wait_flag(const Dev &d, const uint32_t *flag, ui
  * device-scope stores; the waiter reads the subject's state with
  * device-scope loads. */
 __device__ __forceinline__ void wait_subject(const Dev &d, const SweepArgs &a, int x, uint32_t iter) {
-    const int n = d.nchain, G = d.G;
+    const int G = d.G;
     const uint32_t *ready = d.item_ready + (size_t)x * G * a.rmax;
     for (int e = threadIdx.x; e < G * a.rmax; e += blockDim.x) {
-        const int g = e / a.rmax, r = e - g * a.rmax;
-        const int ng = group_lo(g + 1, n, G) - group_lo(g, n, G);
-        if (r < (ng + a.kmax - 1) / a.kmax) wait_flag(d, ready + e, iter);
+        const int g = quo(e, a.by_r), r = e - g * a.rmax;
+        if (r < ranges(d, a, g)) wait_flag(d, ready + e, iter);
     }
     __syncthreads();
 }
@@ -1713,8 +1734,7 @@ __device__ __forceinline__ void wait_run(const Dev &d, const SweepArgs &a, int f
         const uint32_t *ready = d.item_ready + (size_t)job.first_subject * per;
         for (int e = threadIdx.x; e < job.nsubject * per; e += blockDim.x) {
             const int q = e % per, g = q / a.rmax, r = q - g * a.rmax;
-            const int ng = group_lo(g + 1, n, G) - group_lo(g, n, G);
-            if (r < (ng + a.kmax - 1) / a.kmax) wait_flag(d, ready + e, iter);
+            if (r < ranges(d, a, g)) wait_flag(d, ready + e, iter);
         }
     }
     __syncthreads();
@@ -1730,10 +1750,10 @@ __device__ __forceinline__ void wait_chain_run(const Dev &d, const SweepArgs &a,
     const int n = d.nchain, G = d.G;
     const JobDev job = d.phi_jobs[f];
     int g = 0;
-    while (group_lo(g + 1, n, G) <= i) ++g;
+    while (glo(d, g + 1) <= i) ++g;
     const int per = G * a.rmax;
     const uint32_t *ready = d.item_ready + (size_t)job.first_subject * per + (size_t)g * a.rmax +
-                            (i - group_lo(g, n, G)) / a.kmax;
+                            quo(i - glo(d, g), a.by_k);
     const int ns = job.kind == GGDMC_KIND_HIER ? job.nsubject : 0;
     for (int e = threadIdx.x; e < n + ns; e += blockDim.x)
         wait_flag(d, e < n ? d.phi_ready + (size_t)f * n + e : ready + (size_t)(e - n) * per, iter);
@@ -1752,7 +1772,7 @@ __device__ __forceinline__ double load_agent(const double *p) {
 __device__ __forceinline__ void late_prior(const Dev &d, const JobDev &job, const SweepLds &L, int i0, int k) {
     const int P = d.P, n = d.nchain;
     for (int e = threadIdx.x; e < k * P; e += blockDim.x) {
-        const int c = e / P, p = e - c * P;
+        const int c = quo(e, d.by_P), p = e - c * P;
         const size_t r = ((size_t)job.phi_index * n + i0 + c) * P + p;
         const double *ph = d.phi + ((size_t)job.phi_index * n + i0 + c) * (2 * P);
         const double q[4] = {load_agent(ph + p), load_agent(ph + P + p), load_agent(d.pcache + 2 * r),
@@ -1793,8 +1813,8 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
          * per (state, chain); whole-run steps by the first chain's workgroup
          * of the first group */
         const int gb = a.chained ? 0 : a.g_begin, ge = a.chained ? d.G : a.g_end;
-        const int c_lo = group_lo(gb, d.nchain, d.G);
-        const int nc = group_lo(ge, d.nchain, d.G) - c_lo;
+        const int c_lo = glo(d, gb);
+        const int nc = glo(d, ge) - c_lo;
         const int f = wid / nc, i = c_lo + wid % nc;
         const uint32_t it = *d.iter_base + a.iter_off + (uint32_t)seg;
         if (!phi_full(d, d.phi_jobs[f], it)) {
@@ -1894,8 +1914,8 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
     const int para = blocked ? a.sweep : -1;
     const Stream st = make_stream(seed, iter + d.philox_offset, unit, (uint32_t)a.sweep);
     auto group_k = [&](int g, int &lo, int &hi, int &i0) {
-        lo = group_lo(g, n, G);
-        hi = group_lo(g + 1, n, G);
+        lo = glo(d, g);
+        hi = glo(d, g + 1);
         i0 = lo + c0;
         return min(c1 == kAllChains ? hi - lo : c1, hi - lo) - c0;
     };
@@ -1941,8 +1961,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
      * this subject first; then the rows of the earlier groups' chains, which
      * they changed */
     auto wait_prev_group = [&](int gq) {
-        const int glo = group_lo(gq - 1, n, G);
-        const int nr = (group_lo(gq, n, G) - glo + a.kmax - 1) / a.kmax;
+        const int g_lo = glo(d, gq - 1), nr = ranges(d, a, gq - 1);
         if (G == 2 && !a.tiles) {
             /* two groups, whole subjects: every group-0 item of the subject
              * has read its rows, and the items holding this item's partners
@@ -1952,7 +1971,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
             const int k1 = group_k(gq, lo1, hi1, i01);
             for (int e = threadIdx.x; e < 2 * k1; e += blockDim.x) {
                 const int m = (e & 1) ? L.m1[e >> 1] : L.m0[e >> 1];
-                const uint32_t *f = ready + (m - glo) / a.kmax;
+                const uint32_t *f = ready + quo(m - g_lo, a.by_k);
                 uint32_t spins = 0;
                 while (!reached(__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), iter)) {
                     if (++spins == kSpinLimit ||
@@ -1968,7 +1987,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
             wait_items(d, ready + (size_t)(gq - 1) * a.rmax, nr, iter);
         }
         const double *src = d.theta + (size_t)x * n * P;
-        for (int e = threadIdx.x; e < group_lo(gq, n, G) * P; e += blockDim.x)
+        for (int e = threadIdx.x; e < glo(d, gq) * P; e += blockDim.x)
             L.th[e] = __hip_atomic_load(src + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
     };
@@ -1989,9 +2008,8 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
                 __builtin_amdgcn_s_waitcnt(0);
                 __syncthreads();
                 for (int e = threadIdx.x; e < G * a.rmax; e += blockDim.x) {
-                    const int g = e / a.rmax, r = e - g * a.rmax;
-                    const int ng = group_lo(g + 1, n, G) - group_lo(g, n, G);
-                    if (r < (ng + a.kmax - 1) / a.kmax)
+                    const int g = quo(e, a.by_r), r = e - g * a.rmax;
+                    if (r < ranges(d, a, g))
                         __hip_atomic_store(ready + e, iter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
             }
@@ -2262,9 +2280,8 @@ __global__ __launch_bounds__(kBlock) void plain_phi_kernel(Dev d, uint32_t iter,
  * state: the plain path after each iteration, the batched path for the last
  * iteration of an advance (whose subject store is otherwise deferred). */
 __global__ void store_kernel(Dev d, uint32_t iter, int subjects_only) {
-    if (iter % (uint32_t)d.thin != 0) return;
-    const int k = (int)(iter / (uint32_t)d.thin);
-    if (k >= d.nmc) return;
+    int k;
+    if (!stored(d, iter, k)) return;
     const int n = d.nchain, P = d.P;
     const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
