@@ -41,7 +41,7 @@ size_t ggdmc_internal_sweep_lds(int n, int P, int kmax, int per_chain, int chain
                                 int tstage);
 size_t ggdmc_internal_phi_lds(int n, int P, int G, int stats_lds);
 size_t ggdmc_internal_phi_chain_lds(int P, int max_subjects);
-hipError_t ggdmc_internal_launch_sweep(const Dev *d, const SweepArgs *a, int mode, size_t lds, int occ,
+hipError_t ggdmc_internal_launch_sweep(const Dev *d, const SweepArgs *a, int mode, size_t lds, int occ, bool lean,
                                        hipStream_t stream);
 hipError_t ggdmc_internal_launch_phi(const Dev *d, uint32_t iter_off, size_t lds, int stats_lds,
                                      hipStream_t stream);
@@ -231,6 +231,14 @@ struct ggdmc_session {
         bool span;
         int occ;
     };
+    /* every iteration of every run is a plain crossover (the sampling phase):
+     * no migration, blocked sweep, hyper-only run, trial tile or trace */
+    bool lean() const {
+        bool hyper = false;
+        for (const ggdmc_job &j : jobs) hyper = hyper || j.kind == GGDMC_KIND_HYPER;
+        return !hyper && !tiled && !d.trace && !d.blocked_sub && !d.blocked_pop && !(d.sub_mig > 0.0) &&
+               !(d.n_phi > 0 && d.pop_mig > 0.0);
+    }
     std::vector<Decomp> candidates() const;
     bool try_decomp(const Decomp &c);
     bool decomp_given() const {
@@ -859,7 +867,7 @@ void ggdmc_session::enqueue_iteration(uint32_t off, std::vector<hipEvent_t> *ev,
                 ev->push_back(e1);
                 HIPCHECK(hipEventRecord(e0, stream));
             }
-            HIPCHECK(ggdmc_internal_launch_sweep(&d, &a, lk, with_phi ? ovl_lds : sweep_lds, occ, stream));
+            HIPCHECK(ggdmc_internal_launch_sweep(&d, &a, lk, with_phi ? ovl_lds : sweep_lds, occ, lean(), stream));
             if (ev) HIPCHECK(hipEventRecord(e1, stream));
         }
     }

@@ -1480,10 +1480,11 @@ __device__ __forceinline__ void phi_chain(const Dev &d, int f, int i, uint32_t i
     const size_t off = (size_t)f * n;
     const size_t nq = (size_t)n * P;
     const double *tbase = d.theta + (size_t)job.first_subject * nq + (size_t)i * P;
-    /* loads in one batch: the subject values of this chain (one block),
-     * rows i, m0, m1, chain i's cached logarithms, the prior constants */
-    double v[kStatBlock];
-    if (nblk == 1) block_load<AG>(tbase + min(t, P - 1), nq, S, v);
+    /* loads in one batch: row i, its cached logarithms and the prior constants,
+     * then the subject values of this chain, whose statistics every load's
+     * latency overlaps. 2P <= 128 entries: one per thread. One copy of the
+     * moments' code serves runs of one block and of several (the kernel is
+     * larger than the instruction cache). */
     {
         Piece<double, 1, AG> pxi{xi, d.phi + (off + i) * P2, P2};
         Piece<double, 1, AG> ppc{pc, d.pcache + (off + i) * P2, P2};
@@ -1497,6 +1498,20 @@ __device__ __forceinline__ void phi_chain(const Dev &d, int f, int i, uint32_t i
         const double b0 = d.pr_lo[kp], b1 = d.pr_up[kp];
         const double lp0 = ld<AG>(d.phi_lp + off + i);
         const int valid = ld<AG>(d.pcache_valid + off + i);
+#pragma clang loop unroll(disable)
+        for (int e = t; e < P * nblk; e += bs) {
+            const int pr = nblk == 1 ? e : e / nblk, j = e - pr * nblk;
+            const int nb = min(kStatBlock, S - j * kStatBlock);
+            double v[kStatBlock], sum, m2, mn, mx;
+            bool nan;
+            block_load<AG>(tbase + (size_t)j * kStatBlock * nq + pr, nq, nb, v);
+            block_moments(v, nb, sum, m2, mn, mx, nan);
+            double *o = (nblk == 1 ? stt : bst) + (size_t)e * 4;
+            o[0] = nan ? __builtin_nan("") : (nblk == 1 ? sum / (double)S : sum);
+            o[1] = m2;
+            o[2] = mn;
+            o[3] = mx;
+        }
         pxi.store();
         ppc.store();
         if (t < P2) {
@@ -1516,43 +1531,6 @@ __device__ __forceinline__ void phi_chain(const Dev &d, int f, int i, uint32_t i
         if (t == 0) {
             misc[0] = lp0;
             flag[0] = valid;
-        }
-        for (int r = t + bs; r < P2; r += bs) {
-            const int kk = job.hprior_off + r;
-            double *h = L.hc + (size_t)r * 6;
-            h[0] = d.pr_p0[kk];
-            h[1] = d.pr_p1[kk];
-            h[2] = d.pr_lo[kk];
-            h[3] = d.pr_up[kk];
-            h[4] = d.scache[2 * kk];
-            h[5] = d.scache[2 * kk + 1];
-            L.hd[r] = d.pr_dist[kk];
-            if (r < P) {
-                L.sb[2 * r] = d.pr_lo[job.prior_off + r];
-                L.sb[2 * r + 1] = d.pr_up[job.prior_off + r];
-            }
-        }
-    }
-    /* statistics of chain i's values of each parameter */
-    if (nblk == 1) {
-        if (t < P) direct_stats(v, S, stt + (size_t)t * 4);
-        for (int r = t + bs; r < P; r += bs) {
-            block_load<AG>(tbase + r, nq, S, v);
-            direct_stats(v, S, stt + (size_t)r * 4);
-        }
-    } else {
-        for (int e = t; e < P * nblk; e += bs) {
-            const int pr = e / nblk, j = e - pr * nblk;
-            const int nb = min(kStatBlock, S - j * kStatBlock);
-            double sum, m2, mn, mx;
-            bool nan;
-            block_load<AG>(tbase + (size_t)j * kStatBlock * nq + pr, nq, nb, v);
-            block_moments(v, nb, sum, m2, mn, mx, nan);
-            double *o = bst + (size_t)e * 4;
-            o[0] = nan ? __builtin_nan("") : sum;
-            o[1] = m2;
-            o[2] = mn;
-            o[3] = mx;
         }
     }
     __syncthreads();
@@ -1652,21 +1630,23 @@ constexpr uint32_t kSpinLimit = 1u << 18;
  * several iterations in a launch a flag may already hold a later one). */
 __device__ __forceinline__ bool reached(uint32_t v, uint32_t iter) { return (int32_t)(v - iter) >= 0; }
 
+/* One flag, by one thread. */
+__device__ __forceinline__ void wait_flag(const Dev &d, const uint32_t *flag, uint32_t iter) {
+    uint32_t spins = 0;
+    while (!reached(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), iter)) {
+        /* after one failure every later wait gives up at once */
+        if (++spins == kSpinLimit || __hip_atomic_load(d.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+            atomicOr(d.fault, 1u);
+            break;
+        }
+        __builtin_amdgcn_s_sleep(4);
+    }
+}
+
 __device__ __forceinline__ void wait_chains(const Dev &d, int f, int c_lo, int c_n, uint32_t iter,
                                             bool acquire) {
-    for (int c = threadIdx.x; c < c_n; c += blockDim.x) {
-        const uint32_t *flag = d.phi_ready + (size_t)f * d.nchain + c_lo + c;
-        uint32_t spins = 0;
-        while (!reached(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), iter)) {
-            /* after one failure every later wait gives up at once */
-            if (++spins == kSpinLimit ||
-                __hip_atomic_load(d.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                atomicOr(d.fault, 1u);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(4);
-        }
-    }
+    for (int c = threadIdx.x; c < c_n; c += blockDim.x)
+        wait_flag(d, d.phi_ready + (size_t)f * d.nchain + c_lo + c, iter);
     __syncthreads();
     if (acquire) __threadfence();
 }
@@ -1682,30 +1662,8 @@ __device__ __forceinline__ void publish_item(uint32_t *ready, int r, uint32_t it
 
 /* Waits (bounded, as wait_chains) until ready[0..nr) all reach iter. */
 __device__ __forceinline__ void wait_items(const Dev &d, const uint32_t *ready, int nr, uint32_t iter) {
-    for (int r = threadIdx.x; r < nr; r += blockDim.x) {
-        uint32_t spins = 0;
-        while (!reached(__hip_atomic_load(ready + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), iter)) {
-            if (++spins == kSpinLimit ||
-                __hip_atomic_load(d.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                atomicOr(d.fault, 1u);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(4);
-        }
-    }
+    for (int r = threadIdx.x; r < nr; r += blockDim.x) wait_flag(d, ready + r, iter);
     __syncthreads();
-}
-
-/* Bounded wait (as wait_chains) for one flag; false on giving up. */
-__device__ __forceinline__ void wait_flag(const Dev &d, const uint32_t *flag, uint32_t iter) {
-    uint32_t spins = 0;
-    while (!reached(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), iter)) {
-        if (++spins == kSpinLimit || __hip_atomic_load(d.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-            atomicOr(d.fault, 1u);
-            break;
-        }
-        __builtin_amdgcn_s_sleep(4);
-    }
 }
 
 /* Several iterations per launch: every item of subject x (each group's
@@ -1790,10 +1748,29 @@ __device__ __forceinline__ void late_prior(const Dev &d, const JobDev &job, cons
 
 /* ------------------------------------------------------------ sweep kernel */
 /* OCC: waves per SIMD the kernel is built for (3: up to 168 VGPRs a lane, 4:
- * 128, with values of the cold paths in scratch). */
-template <int MODE, bool MULTI, int OCC>
+ * 128, with values of the cold paths in scratch). LEAN: for launches whose every
+ * iteration is a plain crossover of whole subjects (no migration, blocked
+ * sweep, hyper-only run, trial tile or decision trace): without the migration
+ * ring's and the whole-run population step's copies of the code the kernel is 87
+ * KB instead of 230 and its path fits the 64 KB instruction cache of a CU pair
+ * more often, which bounds an iteration of few subjects as much as its
+ * arithmetic (us an iteration, general and lean: 18-chain fit 22.7 and 20.5,
+ * 32 x 768 32.9 and 29.8, FP64 41.0 and 37.7, 256 ragged + 64 fits 144 and
+ * 131, 512 x 2048 of 4 accumulators 308 and 299). */
+template <int MODE, bool MULTI, int OCC, bool LEAN>
 __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, SweepArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
+    /* what the host checked: drops the loops that take a workgroup's second pass */
+    __builtin_assume(blockDim.x == kBlock);
+    __builtin_assume(d.P >= 1 && d.P <= 64);
+    __builtin_assume(d.nchain >= 3 && d.nchain <= kMaxChains);
+    if constexpr (LEAN) {
+        d.trace = nullptr;
+        d.blocked_sub = d.blocked_pop = 0;
+        a.sweep = 0;
+        a.chained = 1;
+        a.tiles = 0;
+    }
     /* several iterations per launch (MULTI): segment seg of seg_wgs
      * workgroups runs iteration base + seg; its workgroups wait only on
      * lower workgroup ids (the previous segment, or earlier in their own),
@@ -1817,7 +1794,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
         const int nc = glo(d, ge) - c_lo;
         const int f = wid / nc, i = c_lo + wid % nc;
         const uint32_t it = *d.iter_base + a.iter_off + (uint32_t)seg;
-        if (!phi_full(d, d.phi_jobs[f], it)) {
+        if (LEAN || !phi_full(d, d.phi_jobs[f], it)) {
             if (MULTI && seg > 0) wait_chain_run(d, a, f, i, it - 1);
             phi_chain<MULTI>(d, f, i, it, lds_raw, a.chained != 0);
         } else if (gb == 0 && i == 0) {
@@ -1834,7 +1811,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
     const int4 item = a.items[ib];
     const int x = item.x;
     const int c0 = item.y >> 16, c1 = item.y & 0xFFFF;
-    const int t = item.z >> 16, ntile = item.z & 0xFFFF;
+    const int t = LEAN ? 0 : item.z >> 16, ntile = LEAN ? 1 : item.z & 0xFFFF;
     const int n = d.nchain, P = d.P, G = d.G;
     /* the item's chain groups [g_begin, g_end) and chain range r */
     const int g_begin = a.chained ? item.w >> 16 : a.g_begin;
@@ -1910,7 +1887,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
     /* level decision (src/de.cpp:208-236 single level, :333-372 subjects) */
     const int dsweep = (blocked && single) ? 0 : a.sweep;
     const Stream sd = make_stream(seed, iter + d.philox_offset, unit, (uint32_t)dsweep);
-    const bool migrate = decision_u(sd) < d.sub_mig;
+    const bool migrate = !LEAN && decision_u(sd) < d.sub_mig;
     const int para = blocked ? a.sweep : -1;
     const Stream st = make_stream(seed, iter + d.philox_offset, unit, (uint32_t)a.sweep);
     auto group_k = [&](int g, int &lo, int &hi, int &i0) {
@@ -1971,16 +1948,7 @@ __global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, Sweep
             const int k1 = group_k(gq, lo1, hi1, i01);
             for (int e = threadIdx.x; e < 2 * k1; e += blockDim.x) {
                 const int m = (e & 1) ? L.m1[e >> 1] : L.m0[e >> 1];
-                const uint32_t *f = ready + quo(m - g_lo, a.by_k);
-                uint32_t spins = 0;
-                while (!reached(__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), iter)) {
-                    if (++spins == kSpinLimit ||
-                        __hip_atomic_load(d.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-                        atomicOr(d.fault, 1u);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(4);
-                }
+                wait_flag(d, ready + quo(m - g_lo, a.by_k), iter);
             }
             __syncthreads();
         } else {
@@ -2448,6 +2416,22 @@ __global__ __launch_bounds__(kLoglikeBlock) void loglike_kernel(Dev d, LoglikeSp
 /* ------------------------------------------------------ launch wrappers */
 using namespace ggdmc;
 
+/* occ (waves per SIMD) 4 and lean exist for several iterations per launch only. */
+template <int MODE>
+static void launch_sweep(const Dev *d, const SweepArgs *a, size_t lds, int occ, bool lean, hipStream_t stream) {
+    const dim3 block(kBlock), multi(a->iters * a->seg_wgs);
+    if (a->iters == 1)
+        subject_sweep_kernel<MODE, false, 3, false><<<dim3(a->phi_wgs + a->n_items), block, lds, stream>>>(*d, *a);
+    else if (lean && occ == 4)
+        subject_sweep_kernel<MODE, true, 4, true><<<multi, block, lds, stream>>>(*d, *a);
+    else if (lean)
+        subject_sweep_kernel<MODE, true, 3, true><<<multi, block, lds, stream>>>(*d, *a);
+    else if (occ == 4)
+        subject_sweep_kernel<MODE, true, 4, false><<<multi, block, lds, stream>>>(*d, *a);
+    else
+        subject_sweep_kernel<MODE, true, 3, false><<<multi, block, lds, stream>>>(*d, *a);
+}
+
 extern "C" {
 
 size_t ggdmc_internal_sweep_lds(int n, int P, int kmax, int per_chain, int chain_batch, int cmax,
@@ -2461,31 +2445,10 @@ size_t ggdmc_internal_phi_chain_lds(int P, int max_subjects) {
     return phi_chain_lds_bytes(P, (max_subjects + kStatBlock - 1) / kStatBlock);
 }
 
-/* occ (waves per SIMD) 4 exists for several iterations per launch only. */
-hipError_t ggdmc_internal_launch_sweep(const Dev *d, const SweepArgs *a, int mode, size_t lds, int occ,
+hipError_t ggdmc_internal_launch_sweep(const Dev *d, const SweepArgs *a, int mode, size_t lds, int occ, bool lean,
                                        hipStream_t stream) {
-    const dim3 block(kBlock);
-    const bool mixed = mode == GGDMC_MIXED_BATCHED;
-    if (a->iters > 1) {
-        const dim3 grid(a->iters * a->seg_wgs);
-        if (occ == 4) {
-            if (mixed)
-                subject_sweep_kernel<MODE_MIXED, true, 4><<<grid, block, lds, stream>>>(*d, *a);
-            else
-                subject_sweep_kernel<MODE_NAIVE, true, 4><<<grid, block, lds, stream>>>(*d, *a);
-        } else {
-            if (mixed)
-                subject_sweep_kernel<MODE_MIXED, true, 3><<<grid, block, lds, stream>>>(*d, *a);
-            else
-                subject_sweep_kernel<MODE_NAIVE, true, 3><<<grid, block, lds, stream>>>(*d, *a);
-        }
-        return hipGetLastError();
-    }
-    const dim3 grid(a->phi_wgs + a->n_items);
-    if (mixed)
-        subject_sweep_kernel<MODE_MIXED, false, 3><<<grid, block, lds, stream>>>(*d, *a);
-    else
-        subject_sweep_kernel<MODE_NAIVE, false, 3><<<grid, block, lds, stream>>>(*d, *a);
+    if (mode == GGDMC_MIXED_BATCHED) launch_sweep<MODE_MIXED>(d, a, lds, occ, lean, stream);
+    else launch_sweep<MODE_NAIVE>(d, a, lds, occ, lean, stream);
     return hipGetLastError();
 }
 
