@@ -32,6 +32,7 @@
 namespace ggdmc {
 
 constexpr int kBlock = 256;        /* threads per workgroup of the sweep kernels */
+constexpr int kWideBlock = 512;    /* ... of their build for launches of few items */
 constexpr int kPhiBlock = 512;     /* threads per workgroup of the population kernel */
 constexpr int kWaves = kBlock / 64;
 constexpr int kMaxChains = 256;    /* chains per run */
@@ -159,6 +160,7 @@ struct SweepArgs {
                              grid is iters segments of seg_wgs workgroups, segment s running
                              iteration *iter_base + iter_off + s */
     int32_t seg_wgs;      /* phi_wgs + n_items rounded up to a multiple of 8 (iters > 1) */
+    int32_t wide;         /* iters > 1: workgroups of kWideBlock threads */
     int32_t span;         /* chained: an item holds its chain range of every group, in group
                              order (items carry group 0); else one group per item */
 };

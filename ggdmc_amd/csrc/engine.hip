@@ -180,6 +180,7 @@ struct ggdmc_session {
     bool span = false;            /* chained: an item holds its chain range of every group */
     int occ = 3;                  /* waves per SIMD of the subject kernel (4: several
                                      iterations per launch only) */
+    bool wide = false;            /* several iterations per launch: 8 waves per workgroup */
     bool tiled = false;           /* some subject's trials split over several items */
     int rmax = 1;                 /* chain ranges per group (item_ready stride) */
     int ovl_stats_lds = 0;
@@ -220,7 +221,7 @@ struct ggdmc_session {
 
     void build(const ggdmc_config *c, const ggdmc_model *model, const ggdmc_job *js, int nj);
     void set_decomp(bool fused_new, int k_new, int tpt_new, bool chained_new = false, int ipl_new = 1,
-                    bool span_new = false, int occ_new = 3);
+                    bool span_new = false, int occ_new = 3, bool wide_new = false);
     void default_decomp();
     /* a work decomposition of the subject launches */
     struct Decomp {
@@ -230,6 +231,7 @@ struct ggdmc_session {
         int ipl;
         bool span;
         int occ;
+        bool wide;
     };
     /* every iteration of every run is a plain crossover (the sampling phase):
      * no migration, blocked sweep, hyper-only run, trial tile or trace */
@@ -689,7 +691,7 @@ void ggdmc_session::default_decomp() {
  * (rounded up to a multiple of kChunk; 0 = whole subject); or, fused, one
  * item per subject that sweeps every group in one launch. Sizes the LDS. */
 void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chained_new, int ipl_new,
-                               bool span_new, int occ_new) {
+                               bool span_new, int occ_new, bool wide_new) {
     if (tpt_new > 0) tpt_new = ((tpt_new + kChunk - 1) / kChunk) * kChunk;
     require(!fused_new || tpt_new == 0, "one item per subject needs whole subjects");
     require(!(fused_new && chained_new), "one item per subject already covers every group");
@@ -704,6 +706,7 @@ void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chai
     ipl = ipl_new;
     span = span_new;
     occ = ipl_new > 1 ? occ_new : 3;
+    wide = wide_new && ipl_new > 1;
     tiled = false;
     tpt = tpt_new;
     d.tpt = tpt;
@@ -858,7 +861,7 @@ void ggdmc_session::enqueue_iteration(uint32_t off, std::vector<hipEvent_t> *ev,
             const int seg_wgs = multi > 1 ? (pw + list_n[g] + 7) / 8 * 8 : pw + list_n[g];
             SweepArgs a{off, sw, (fused || chained) ? 0 : g, (fused || chained) ? d.G : g + 1, (int)store,
                         chain_batch, kmax, cmax, tstage, list_n[g], lists[g],
-                        pw, ovl_stats_lds, (int)chained, rmax, fast_div(kmax), fast_div(rmax), (int)tiled, multi, seg_wgs, (int)span};
+                        pw, ovl_stats_lds, (int)chained, rmax, fast_div(kmax), fast_div(rmax), (int)tiled, multi, seg_wgs, (int)wide, (int)span};
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (ev) {
                 HIPCHECK(hipEventCreate(&e0));
@@ -980,7 +983,7 @@ void ggdmc_session::run_plain(uint32_t n_iter) {
 
 bool ggdmc_session::try_decomp(const Decomp &c) {
     try {
-        set_decomp(c.fused, c.k, c.tpt, c.chained, c.ipl, c.span, c.occ);
+        set_decomp(c.fused, c.k, c.tpt, c.chained, c.ipl, c.span, c.occ, c.wide);
     } catch (const Error &) {
         if (c.ipl == 1) throw;
         return false;   /* no population step inside the launch for this design */
@@ -1030,7 +1033,7 @@ std::vector<ggdmc_session::Decomp> ggdmc_session::candidates() const {
     auto add = [&](const Decomp &c) {
         for (const Decomp &o : out)
             if (o.fused == c.fused && o.k == c.k && o.tpt == c.tpt && o.chained == c.chained && o.ipl == c.ipl &&
-                o.span == c.span && o.occ == c.occ)
+                o.span == c.span && o.occ == c.occ && o.wide == c.wide)
                 return;
         out.push_back(c);
     };
@@ -1043,32 +1046,41 @@ std::vector<ggdmc_session::Decomp> ggdmc_session::candidates() const {
     const bool can_chain = nsweep_sub == 1 && cfg.launch_mode != 1 &&
                            rounds * chunk_us * std::max(k, d.sub_mig > 0.0 ? d.nchain : 1) < 5e4;
     if (can_chain) {
-        auto multi = [&](int kk, bool span, int oc) {
+        /* 8 waves per workgroup where every workgroup of two segments has a CU
+         * to itself and 4 waves would take an item's chunks in several rounds
+         * (1 x 768, 6 chunks: 18 chains 20.5 -> 19.1 us an iteration; 39 chains
+         * in FP64 with migration rings 49.5 -> 41 us) */
+        const int pw = d.n_phi > 0 ? d.n_phi * d.nchain : 0;
+        auto few = [&](int kk) {
+            return cfg.waves_per_simd == 0 && 2 * (items(kk) + pw) <= cus && max_ntr * kk > kChunk * kWaves;
+        };
+        auto multi = [&](int kk, bool span, int oc, bool wide = false) {
             if (cfg.waves_per_simd != 0) oc = cfg.waves_per_simd;
             if (span && !span_fits((ng + kk - 1) / kk)) span = false;
-            add({false, kk, 0, true, kItersPerLaunch, span, oc});
+            add({false, kk, 0, true, kItersPerLaunch, span, oc, wide});
         };
         const bool span = k == 1 || k == ng;
         if (items(1) <= cus && max_ntr >= 2048) {
-            add({false, std::min(2, ng), 256, true, 1, false, 3});
-            add({false, 1, 256, true, 1, false, 3});
+            add({false, std::min(2, ng), 256, true, 1, false, 3, false});
+            add({false, 1, 256, true, 1, false, 3, false});
         }
+        if (few(k)) multi(k, span, 3, true);
         multi(k, span, occ);
-        if (d.G > 2) add({true, 0, 0, false, 1, false, 3});
+        if (d.G > 2) add({true, 0, 0, false, 1, false, 3, false});
         multi(k, !span, occ);
         multi(k, span, 7 - occ);
         if (i + 1 < ks.size()) multi(ks[i + 1], false, 3);
         if (i > 0) multi(ks[i - 1], false, 4);
         if (i > 0) multi(ks[i - 1], true, 4);
-        if (items(1) <= cus && max_ntr > 1024) add({false, 1, 1024, true, 1, false, 3});
-        add({false, k, 0, true, 1, false, 3});
+        if (items(1) <= cus && max_ntr > 1024) add({false, 1, 1024, true, 1, false, 3, false});
+        add({false, k, 0, true, 1, false, 3, false});
     }
-    add({false, k, 0, false, 1, false, 3});
+    add({false, k, 0, false, 1, false, 3, false});
     if (!can_chain) {
-        add({true, 0, 0, false, 1, false, 3});
-        if (i + 1 < ks.size()) add({false, ks[i + 1], 0, false, 1, false, 3});
-        if (items(1) <= cus && max_ntr > 256) add({false, k, 256, false, 1, false, 3});
-        if (i > 0) add({false, ks[i - 1], 0, false, 1, false, 3});
+        add({true, 0, 0, false, 1, false, 3, false});
+        if (i + 1 < ks.size()) add({false, ks[i + 1], 0, false, 1, false, 3, false});
+        if (items(1) <= cus && max_ntr > 256) add({false, k, 256, false, 1, false, 3, false});
+        if (i > 0) add({false, ks[i - 1], 0, false, 1, false, 3, false});
     }
     return out;
 }
@@ -1222,7 +1234,7 @@ void ggdmc_session::autotune() {
         }
     }
     next_iter = it0;
-    set_decomp(pick.fused, pick.k, pick.tpt, pick.chained, pick.ipl, pick.span, pick.occ);
+    try_decomp(pick);
 }
 
 static int fail(const std::exception &e) {

@@ -1747,7 +1747,9 @@ __device__ __forceinline__ void late_prior(const Dev &d, const JobDev &job, cons
 }
 
 /* ------------------------------------------------------------ sweep kernel */
-/* OCC: waves per SIMD the kernel is built for (3: up to 168 VGPRs a lane, 4:
+/* BLOCK: 512 (8 waves, at most one workgroup a CU) where the items are few and
+ * hold more chunks than 4 waves take at once. OCC: waves per SIMD the kernel is
+ * built for (3: up to 168 VGPRs a lane, 4:
  * 128, with values of the cold paths in scratch). LEAN: for launches whose every
  * iteration is a plain crossover of whole subjects (no migration, blocked
  * sweep, hyper-only run, trial tile or decision trace): without the migration
@@ -1757,11 +1759,11 @@ __device__ __forceinline__ void late_prior(const Dev &d, const JobDev &job, cons
  * arithmetic (us an iteration, general and lean: 18-chain fit 22.7 and 20.5,
  * 32 x 768 32.9 and 29.8, FP64 41.0 and 37.7, 256 ragged + 64 fits 144 and
  * 131, 512 x 2048 of 4 accumulators 308 and 299). */
-template <int MODE, bool MULTI, int OCC, bool LEAN>
-__global__ __launch_bounds__(kBlock, OCC) void subject_sweep_kernel(Dev d, SweepArgs a) {
+template <int MODE, bool MULTI, int OCC, bool LEAN, int BLOCK = kBlock>
+__global__ __launch_bounds__(BLOCK, OCC) void subject_sweep_kernel(Dev d, SweepArgs a) {
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
     /* what the host checked: drops the loops that take a workgroup's second pass */
-    __builtin_assume(blockDim.x == kBlock);
+    __builtin_assume(blockDim.x == BLOCK);
     __builtin_assume(d.P >= 1 && d.P <= 64);
     __builtin_assume(d.nchain >= 3 && d.nchain <= kMaxChains);
     if constexpr (LEAN) {
@@ -2419,8 +2421,12 @@ using namespace ggdmc;
 /* occ (waves per SIMD) 4 and lean exist for several iterations per launch only. */
 template <int MODE>
 static void launch_sweep(const Dev *d, const SweepArgs *a, size_t lds, int occ, bool lean, hipStream_t stream) {
-    const dim3 block(kBlock), multi(a->iters * a->seg_wgs);
-    if (a->iters == 1)
+    const dim3 block(kBlock), multi(a->iters * a->seg_wgs), wide(kWideBlock);
+    if (a->iters > 1 && a->wide && lean)
+        subject_sweep_kernel<MODE, true, 2, true, kWideBlock><<<multi, wide, lds, stream>>>(*d, *a);
+    else if (a->iters > 1 && a->wide)
+        subject_sweep_kernel<MODE, true, 2, false, kWideBlock><<<multi, wide, lds, stream>>>(*d, *a);
+    else if (a->iters == 1)
         subject_sweep_kernel<MODE, false, 3, false><<<dim3(a->phi_wgs + a->n_items), block, lds, stream>>>(*d, *a);
     else if (lean && occ == 4)
         subject_sweep_kernel<MODE, true, 4, true><<<multi, block, lds, stream>>>(*d, *a);
