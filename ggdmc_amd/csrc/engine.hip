@@ -87,27 +87,64 @@ void require(bool ok, const std::string &msg) {
 
 __global__ void set_base_kernel(uint32_t *p, uint32_t v) { *p = v; }
 
-/* Device memory owned by a session; freed with it. */
+/* Device memory owned by a session; freed with it. Arrays below 1 MB share
+ * slabs of 2 MB, and uploads below 64 KB are collected in a host copy of their
+ * slab that flush() sends in one transfer (about 45 allocations and 25 transfers
+ * of a few KB each made half a millisecond of a small run). */
 struct Pool {
+    static constexpr size_t kSlab = (size_t)2 << 20, kOwn = (size_t)1 << 20, kSmallUpload = (size_t)64 << 10,
+                            kUploadSlab = (size_t)256 << 10;
     std::vector<void *> ptrs;
+    char *slab = nullptr, *up = nullptr;   /* the current slabs */
+    size_t used = kSlab, up_used = kUploadSlab, up_sent = kUploadSlab;
+    std::vector<char> up_host;
+
+    void *raw(size_t bytes) {
+        void *p = nullptr;
+        HIPCHECK(hipMalloc(&p, bytes));
+        ptrs.push_back(p);
+        return p;
+    }
+    static size_t align(size_t x) { return (std::max<size_t>(x, 1) + 255) & ~(size_t)255; }
     template <class T>
     T *alloc(size_t n) {
-        void *p = nullptr;
-        if (n == 0) n = 1;
-        HIPCHECK(hipMalloc(&p, n * sizeof(T)));
-        ptrs.push_back(p);
-        return static_cast<T *>(p);
+        const size_t bytes = align(n * sizeof(T));
+        if (bytes >= kOwn) return static_cast<T *>(raw(bytes));
+        if (used + bytes > kSlab) {
+            slab = static_cast<char *>(raw(kSlab));
+            used = 0;
+        }
+        char *p = slab + used;
+        used += bytes;
+        return reinterpret_cast<T *>(p);
     }
-    /* The copy has completed when this returns: callers pass host vectors
-     * that may go out of scope right after. */
+    /* The vector may go out of scope once this returns; the device copy is
+     * complete after flush(). */
     template <class T>
     T *upload(const std::vector<T> &v, hipStream_t st) {
-        T *p = alloc<T>(v.size());
-        if (!v.empty()) {
-            HIPCHECK(hipMemcpyAsync(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, st));
+        const size_t bytes = v.size() * sizeof(T);
+        if (bytes >= kSmallUpload) {
+            T *p = alloc<T>(v.size());
+            HIPCHECK(hipMemcpyAsync(p, v.data(), bytes, hipMemcpyHostToDevice, st));
             HIPCHECK(hipStreamSynchronize(st));
+            return p;
         }
+        if (up_used + align(bytes) > kUploadSlab) {
+            flush(st);
+            up = static_cast<char *>(raw(kUploadSlab));
+            up_used = up_sent = 0;
+            up_host.resize(kUploadSlab);
+        }
+        if (bytes) std::memcpy(up_host.data() + up_used, v.data(), bytes);
+        T *p = reinterpret_cast<T *>(up + up_used);
+        up_used += align(bytes);
         return p;
+    }
+    void flush(hipStream_t st) {
+        if (up_sent >= up_used) return;
+        HIPCHECK(hipMemcpyAsync(up + up_sent, up_host.data() + up_sent, up_used - up_sent, hipMemcpyHostToDevice, st));
+        HIPCHECK(hipStreamSynchronize(st));
+        up_sent = up_used;
     }
     ~Pool() {
         for (void *p : ptrs) (void)hipFree(p);
@@ -201,8 +238,6 @@ struct ggdmc_session {
     double *hyper_rows = nullptr;
     int64_t *hyper_off = nullptr;
     std::vector<int64_t> subj_ntr;   /* host copy of trial counts */
-    std::vector<int> subj_of_job;    /* first subject of each job */
-    std::vector<int> phi_of_job;
     int64_t max_ntr = 0;
     std::vector<double> hyper_rows_h;
     std::vector<ggdmc_trace_record> trace;   /* decisions of the last advance, ordered */
@@ -430,11 +465,10 @@ void ggdmc_session::build(const ggdmc_config *c, const ggdmc_model *model, const
                 "cell_off must start at 0 and end at ntrial");
         for (int cidx = 0; cidx < model->n_cell; ++cidx) {
             require(sb->cell_off[cidx + 1] >= sb->cell_off[cidx], "cell_off must be non-decreasing");
-            for (int64_t i = sb->cell_off[cidx]; i < sb->cell_off[cidx + 1]; ++i) {
-                rt.push_back(sb->rt[i]);
-                tcode.push_back((uint16_t)((cond.cond_of_cell[cidx] << 3) | model->winner[cidx]));
-            }
+            tcode.insert(tcode.end(), (size_t)(sb->cell_off[cidx + 1] - sb->cell_off[cidx]),
+                         (uint16_t)((cond.cond_of_cell[cidx] << 3) | model->winner[cidx]));
         }
+        rt.insert(rt.end(), sb->rt, sb->rt + sb->ntrial);
         subj_off.push_back((int64_t)rt.size());
         subj_job.push_back(job);
         subj_unit.push_back(unit);
@@ -452,7 +486,6 @@ void ggdmc_session::build(const ggdmc_config *c, const ggdmc_model *model, const
         J.gamma = cfg.gamma_precursor / std::sqrt(2.0 * npde);
         J.first_subject = (int)subj_job.size();
         J.phi_index = -1;
-        subj_of_job.push_back(J.first_subject);
         if (j.kind == GGDMC_KIND_SUBJECT) {
             check_prior(j.p_prior, P, "p_prior");
             require(j.subjects && j.subject_starts && j.subject_outs, "subject run needs data, start, out");
@@ -487,7 +520,6 @@ void ggdmc_session::build(const ggdmc_config *c, const ggdmc_model *model, const
                 hyper_rows_h.insert(hyper_rows_h.end(), j.hyper_data, j.hyper_data + (size_t)j.nsubject * P);
             }
         }
-        phi_of_job.push_back(J.phi_index);
         jd.push_back(J);
     }
 
@@ -621,7 +653,8 @@ void ggdmc_session::build(const ggdmc_config *c, const ggdmc_model *model, const
     hyper_rows = pool.upload(hyper_rows_h, stream);
     hyper_off = pool.upload(hyper_off_h, stream);
 
-    /* outputs, column 0 = start state */
+    /* outputs; column 0 = start state, stored by one launch (a copy per subject
+     * and array took 14 ms of a 1024-subject run) */
     const size_t nmc = (size_t)cfg.nmc;
     d.out_theta = pool.alloc<double>(std::max<size_t>((size_t)S * nmc * n * P, 1));
     d.out_lp = pool.alloc<double>(std::max<size_t>((size_t)S * nmc * n, 1));
@@ -629,22 +662,8 @@ void ggdmc_session::build(const ggdmc_config *c, const ggdmc_model *model, const
     d.phi_out_theta = pool.alloc<double>(std::max<size_t>((size_t)F * nmc * n * 2 * P, 1));
     d.phi_out_lp = pool.alloc<double>(std::max<size_t>((size_t)F * nmc * n, 1));
     d.phi_out_ll = pool.alloc<double>(std::max<size_t>((size_t)F * nmc * n, 1));
-    for (int s = 0; s < S; ++s) {
-        HIPCHECK(hipMemcpyAsync(d.out_theta + (size_t)s * nmc * n * P, d.theta + (size_t)s * n * P,
-                                sizeof(double) * n * P, hipMemcpyDeviceToDevice, stream));
-        HIPCHECK(hipMemcpyAsync(d.out_lp + (size_t)s * nmc * n, d.lp + (size_t)s * n, sizeof(double) * n,
-                                hipMemcpyDeviceToDevice, stream));
-        HIPCHECK(hipMemcpyAsync(d.out_ll + (size_t)s * nmc * n, d.ll + (size_t)s * n, sizeof(double) * n,
-                                hipMemcpyDeviceToDevice, stream));
-    }
-    for (int f = 0; f < F; ++f) {
-        HIPCHECK(hipMemcpyAsync(d.phi_out_theta + (size_t)f * nmc * n * 2 * P, d.phi + (size_t)f * n * 2 * P,
-                                sizeof(double) * n * 2 * P, hipMemcpyDeviceToDevice, stream));
-        HIPCHECK(hipMemcpyAsync(d.phi_out_lp + (size_t)f * nmc * n, d.phi_lp + (size_t)f * n, sizeof(double) * n,
-                                hipMemcpyDeviceToDevice, stream));
-        HIPCHECK(hipMemcpyAsync(d.phi_out_ll + (size_t)f * nmc * n, d.phi_ll + (size_t)f * n, sizeof(double) * n,
-                                hipMemcpyDeviceToDevice, stream));
-    }
+    pool.flush(stream);
+    HIPCHECK(ggdmc_internal_launch_store(&d, 0, 0, stream));
     for (int f = 0; f < F; ++f) {
         const ggdmc_job &j = jobs[phi_job[f]];
         if (j.kind == GGDMC_KIND_HYPER)
@@ -1431,31 +1450,38 @@ int ggdmc_session_download(ggdmc_session *s) {
     try {
         const size_t nmc = (size_t)s->cfg.nmc, n = (size_t)s->d.nchain, P = (size_t)s->d.P;
         HIPCHECK(hipStreamSynchronize(s->stream));
-        for (size_t ji = 0; ji < s->jobs.size(); ++ji) {
-            const ggdmc_job &j = s->jobs[ji];
-            const int f = s->phi_of_job[ji];
-            if (f >= 0) {
-                ggdmc_samples *o = j.phi_out;
-                HIPCHECK(hipMemcpy(o->theta, s->d.phi_out_theta + (size_t)f * nmc * n * 2 * P,
-                                   sizeof(double) * nmc * n * 2 * P, hipMemcpyDeviceToHost));
-                HIPCHECK(hipMemcpy(o->lp, s->d.phi_out_lp + (size_t)f * nmc * n, sizeof(double) * nmc * n,
-                                   hipMemcpyDeviceToHost));
-                HIPCHECK(hipMemcpy(o->ll, s->d.phi_out_ll + (size_t)f * nmc * n, sizeof(double) * nmc * n,
-                                   hipMemcpyDeviceToHost));
-            }
+        /* the caller's buffers of every population state and subject, in the
+         * device arrays' order */
+        std::vector<ggdmc_samples *> phis, subs;
+        for (const ggdmc_job &j : s->jobs) {
+            if (j.kind != GGDMC_KIND_SUBJECT) phis.push_back(j.phi_out);
             if (j.kind == GGDMC_KIND_HYPER) continue;
             const int ns = j.kind == GGDMC_KIND_SUBJECT ? 1 : j.nsubject;
-            for (int k = 0; k < ns; ++k) {
-                const size_t sg = (size_t)s->subj_of_job[ji] + k;
-                ggdmc_samples *o = &j.subject_outs[k];
-                HIPCHECK(hipMemcpy(o->theta, s->d.out_theta + sg * nmc * n * P, sizeof(double) * nmc * n * P,
-                                   hipMemcpyDeviceToHost));
-                HIPCHECK(hipMemcpy(o->lp, s->d.out_lp + sg * nmc * n, sizeof(double) * nmc * n,
-                                   hipMemcpyDeviceToHost));
-                HIPCHECK(hipMemcpy(o->ll, s->d.out_ll + sg * nmc * n, sizeof(double) * nmc * n,
-                                   hipMemcpyDeviceToHost));
-            }
+            for (int k = 0; k < ns; ++k) subs.push_back(&j.subject_outs[k]);
         }
+        std::unique_ptr<char[]> buf;
+        /* one transfer per buffer, or (below 256 KB each, where its fixed cost
+         * of about 10 us dominates) per 16 MB of them through a host buffer:
+         * 3072 transfers took 30 ms of a 1024-subject run */
+        auto get = [&](const std::vector<ggdmc_samples *> &outs, double *ggdmc_samples::*field, const double *src,
+                       size_t doubles) {
+            const size_t bytes = doubles * sizeof(double), most = (size_t)16 << 20;
+            const size_t batch = outs.size() < 2 || bytes >= ((size_t)256 << 10) ? 1 : most / bytes;
+            if (batch > 1 && !buf) buf.reset(new char[most]);
+            for (size_t k = 0; k < outs.size(); k += batch) {
+                const size_t m = std::min(batch, outs.size() - k);
+                char *to = batch > 1 ? buf.get() : reinterpret_cast<char *>(outs[k]->*field);
+                HIPCHECK(hipMemcpy(to, src + k * doubles, m * bytes, hipMemcpyDeviceToHost));
+                if (batch > 1)
+                    for (size_t q = 0; q < m; ++q) std::memcpy(outs[k + q]->*field, to + q * bytes, bytes);
+            }
+        };
+        get(phis, &ggdmc_samples::theta, s->d.phi_out_theta, nmc * n * 2 * P);
+        get(phis, &ggdmc_samples::lp, s->d.phi_out_lp, nmc * n);
+        get(phis, &ggdmc_samples::ll, s->d.phi_out_ll, nmc * n);
+        get(subs, &ggdmc_samples::theta, s->d.out_theta, nmc * n * P);
+        get(subs, &ggdmc_samples::lp, s->d.out_lp, nmc * n);
+        get(subs, &ggdmc_samples::ll, s->d.out_ll, nmc * n);
     } catch (const std::exception &e) {
         return fail(e);
     }

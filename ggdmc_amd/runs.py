@@ -123,26 +123,47 @@ class Posterior:
                 self.log_likelihoods[:, -1].copy())
 
 
-def _state(keep, theta, lp, ll):
-    th = keep.arr(np.asarray(theta, float).T, np.float64)   # [nchain][P] == R [P x nchain]
-    a = keep.arr(lp, np.float64)
-    b = keep.arr(ll, np.float64)
-    st = _lib.State(ptr(th), ptr(a), ptr(b))
-    keep.items.append(st)
-    return st
+def _addr(a):
+    return a.__array_interface__["data"][0]
 
 
-class _Out:
-    def __init__(self, keep, P, nchain, nmc):
-        self.th = np.empty((nmc, nchain, P))
-        self.lp = np.empty((nmc, nchain))
-        self.ll = np.empty((nmc, nchain))
+def _table(keep, rows, struct):
+    """Rows of three 8-byte fields as a C array of struct (a ctypes object per
+    field took most of the assembly of a batch of many subjects)."""
+    t = keep.arr(np.array(rows, np.int64).reshape(len(rows), 3), np.int64)
+    return C.cast(C.c_void_p(_addr(t)), C.POINTER(struct))
+
+
+def _subjects(keep, subjects):
+    rows = []
+    for s in subjects:
+        rt, off = keep.arr(s.rt, np.float64), keep.arr(s.cell_off, np.int64)
+        rows.append((len(rt), _addr(rt), _addr(off)))
+    return _table(keep, rows, _lib.Subject)
+
+
+def _states(keep, states):
+    rows = []
+    for theta, lp, ll in states:   # theta [nchain][P] == R [P x nchain]
+        rows.append(tuple(_addr(keep.arr(a, np.float64)) for a in (np.asarray(theta, float).T, lp, ll)))
+    return _table(keep, rows, _lib.State)
+
+
+class _Outs:
+    """Stored samples of m states: one block per array, state by state."""
+
+    def __init__(self, keep, m, P, nchain, nmc):
+        self.th = np.empty((m, nmc, nchain, P))
+        self.lp = np.empty((m, nmc, nchain))
+        self.ll = np.empty((m, nmc, nchain))
         keep.items.extend([self.th, self.lp, self.ll])
-        self.c = _lib.Samples(ptr(self.th), ptr(self.lp), ptr(self.ll))
+        base = np.array([_addr(self.th), _addr(self.lp), _addr(self.ll)], np.int64)
+        step = np.array([self.th.strides[0], self.lp.strides[0], self.ll.strides[0]], np.int64)
+        self.c = _table(keep, base + np.arange(m)[:, None] * step, _lib.Samples)
 
-    def posterior(self, cfg, pnames=None):
-        return Posterior(self.th.transpose(2, 1, 0).copy(), self.lp.T.copy(), self.ll.T.copy(),
-                         cfg.nmc, cfg.thin, cfg.nchain, list(pnames or []))
+    def posteriors(self, cfg, pnames=None):
+        return [Posterior(th.transpose(2, 1, 0).copy(), lp.T.copy(), ll.T.copy(), cfg.nmc, cfg.thin, cfg.nchain,
+                          list(pnames or [])) for th, lp, ll in zip(self.th, self.lp, self.ll)]
 
 
 def make_config(nmc, nchain, thin=1, pop_migration_prob=0.0, sub_migration_prob=0.0,
@@ -227,40 +248,28 @@ class _Batch:
             cj.seed = int(j.seed) & 0xFFFFFFFFFFFFFFFF
             cj.nparameter_de = int(j.nparameter_de)
             cj.p_prior = C.pointer(j.p_prior.c_struct(k))
-            o = {"phi": None, "subjects": []}
+            o = {"phi": None, "subjects": None}
             if j.kind == _lib.KIND_SUBJECT:
-                subs = (_lib.Subject * 1)(j.subject.c_struct(k))
-                sts = (_lib.State * 1)(_state(k, *j.start))
-                out = _Out(k, P, cfg.nchain, cfg.nmc)
-                outs = (_lib.Samples * 1)(out.c)
-                k.items.extend([subs, sts, outs])
-                cj.nsubject = 1
-                cj.subjects = subs
-                cj.subject_starts = sts
-                cj.subject_outs = outs
-                o["subjects"].append(out)
+                subjects, starts = [j.subject], [j.start]
             else:
                 cj.h_prior = C.pointer(j.h_prior.c_struct(k))
-                cj.phi_start = C.pointer(_state(k, *j.phi_start))
-                pout = _Out(k, 2 * P, cfg.nchain, cfg.nmc)
-                cj.phi_out = C.pointer(pout.c)
-                o["phi"] = pout
-                if j.kind == _lib.KIND_HIER:
-                    S = len(j.subjects)
-                    subs = (_lib.Subject * S)(*[s.c_struct(k) for s in j.subjects])
-                    sts = (_lib.State * S)(*[_state(k, *st) for st in j.subject_starts])
-                    outs_l = [_Out(k, P, cfg.nchain, cfg.nmc) for _ in range(S)]
-                    outs = (_lib.Samples * S)(*[x.c for x in outs_l])
-                    k.items.extend([subs, sts, outs])
-                    cj.nsubject = S
-                    cj.subjects = subs
-                    cj.subject_starts = sts
-                    cj.subject_outs = outs
-                    o["subjects"] = outs_l
-                else:
-                    hd = k.arr(j.hyper_data, np.float64)
-                    cj.nsubject = hd.shape[0]
-                    cj.hyper_data = ptr(hd)
+                cj.phi_start = _states(k, [j.phi_start])
+                o["phi"] = _Outs(k, 1, 2 * P, cfg.nchain, cfg.nmc)
+                cj.phi_out = o["phi"].c
+                subjects, starts = j.subjects, j.subject_starts
+            if j.kind == _lib.KIND_HYPER:
+                hd = k.arr(j.hyper_data, np.float64)
+                cj.nsubject = hd.shape[0]
+                cj.hyper_data = ptr(hd)
+            else:
+                S = len(subjects)
+                if len(starts) != S:
+                    raise ValueError("%d start states for %d subjects" % (len(starts), S))
+                cj.nsubject = S
+                cj.subjects = _subjects(k, subjects)
+                cj.subject_starts = _states(k, starts)
+                o["subjects"] = _Outs(k, S, P, cfg.nchain, cfg.nmc)
+                cj.subject_outs = o["subjects"].c
             self.outs.append(o)
         k.items.extend([self.cmodel, cjobs])
 
@@ -272,9 +281,9 @@ class _Batch:
         """Per job {'phi': Posterior|None, 'subjects': [Posterior]}."""
         res = []
         for j, o in zip(self.jobs, self.outs):
-            res.append({"phi": o["phi"].posterior(self.cfg, j.h_prior.pnames if j.h_prior else None)
-                        if o["phi"] is not None else None,
-                        "subjects": [x.posterior(self.cfg, j.p_prior.pnames) for x in o["subjects"]]})
+            phi, subs = o["phi"], o["subjects"]
+            res.append({"phi": phi.posteriors(self.cfg, j.h_prior.pnames if j.h_prior else None)[0] if phi else None,
+                        "subjects": subs.posteriors(self.cfg, j.p_prior.pnames) if subs else []})
         return res
 
 

@@ -46,3 +46,22 @@ def test_one_shot_run_of_one_long_subject(gpu):
     s.advance(s.total_iters)
     _same(got, s.download())
     s.close()
+
+
+def test_stored_samples_reach_their_buffers(gpu):
+    # transfers of 499 KB a subject go straight to its buffer, of 25 KB through
+    # the shared host buffer; 300 fits of 55 KB fill that buffer more than once
+    w = W.make("c3", scale=0.1)
+    few = gpu.run_batch(gpu.make_config(20, w.nchain), w.model, w.jobs)[0]
+    many = gpu.run_batch(gpu.make_config(123, w.nchain), w.model, w.jobs)[0]
+    for p, q in zip(few["subjects"] + [few["phi"]], many["subjects"] + [many["phi"]]):
+        assert np.array_equal(p.theta, q.theta[:, :, :20])
+        assert np.array_equal(p.summed_log_prior, q.summed_log_prior[:, :20])
+        assert np.array_equal(p.log_likelihoods, q.log_likelihoods[:, :20])
+    w = W.make("c1")
+    j = w.jobs[0]
+    jobs = [gpu.JobSpec(gpu.KIND_SUBJECT, 100 + r, j.p_prior, start=j.start, subject=j.subject) for r in range(300)]
+    cfg = gpu.make_config(64, 18)
+    a, b = gpu.run_batch(cfg, w.model, jobs), gpu.run_batch(cfg, w.model, jobs[280:])
+    _same(a[280:], b)
+    assert len({x["subjects"][0].theta[0, 0, -1] for x in a}) > 100
