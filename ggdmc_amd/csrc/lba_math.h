@@ -170,6 +170,17 @@ inline void fill_exp2_table(double *t) {
     for (int j = 0; j < 64; ++j) t[j] = (double)std::exp2((long double)j / 64.0L);
 }
 
+/* The Mills-ratio coefficients: kMills, or Ops's copy of them (the kernels keep
+ * one in constant memory). */
+template <class Ops>
+GGDMC_FN auto mills_coefs(int) -> decltype(Ops::mills_coefs()) {
+    return Ops::mills_coefs();
+}
+template <class Ops>
+GGDMC_FN const double *mills_coefs(long) {
+    return kMills;
+}
+
 /* e = exp(-z^2/2) and qa = Q(|z|), the upper normal tail beyond |z|, given
  * t = 1/(1 + 0.2625 |z|) (NaN for a NaN t). */
 template <class Ops>
@@ -179,9 +190,10 @@ GGDMC_FN void mixed_tail_t(double z, double t, double &e, double &qa) {
      * coefficient (a scalar register), so no coefficient is first moved into
      * vector registers; the two trials and two tails a lane evaluates give the
      * dependency chains to interleave */
-    double h = kMills[kMillsDeg];
+    const double *c = mills_coefs<Ops>(0);
+    double h = c[kMillsDeg];
 #pragma unroll
-    for (int j = kMillsDeg - 1; j >= 0; --j) h = std::fma(t, h, kMills[j]);
+    for (int j = kMillsDeg - 1; j >= 0; --j) h = std::fma(t, h, c[j]);
     qa = e * (t * h);
 }
 
