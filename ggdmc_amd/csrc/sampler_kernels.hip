@@ -139,15 +139,19 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-/* Sum over the 8 lanes of an aligned lane group (fixed xor tree). */
+/* Sum over the 8 lanes of an aligned lane group, valid in its first four lanes:
+ * the xor tree of strides 4, 2, 1 by DPP moves (lane i takes lane i + 4, then
+ * within quads); as ds_bpermute the three steps were 0.15 us of the chain of a
+ * proposal's sums. */
 __device__ __forceinline__ double sum8(double v) {
-#pragma unroll
-    for (int off = 4; off > 0; off >>= 1) v += __shfl_xor(v, off, 8);
+    v += dpp_f64<0x104>(v);   /* row_shl:4 */
+    v += dpp_f64<0x4E>(v);    /* quad_perm [2,3,0,1] */
+    v += dpp_f64<0xB1>(v);    /* quad_perm [1,0,3,2] */
     return v;
 }
 
 /* Terms t[0..m) summed by 8 lanes (lane l takes terms l, l + 8, ... in order,
- * then the xor tree); every lane of the group gets the sum. */
+ * then the xor tree); the group's first lane gets the sum. */
 __device__ __forceinline__ double group8_sum(const double *t, int m, int l) {
     double v = 0.0;
     for (int q = l; q < m; q += 8) v += t[q];
