@@ -255,8 +255,6 @@ struct ggdmc_session {
     }
 
     void build(const ggdmc_config *c, const ggdmc_model *model, const ggdmc_job *js, int nj);
-    void set_decomp(bool fused_new, int k_new, int tpt_new, bool chained_new = false, int ipl_new = 1,
-                    bool span_new = false, int occ_new = 3, bool wide_new = false);
     void default_decomp();
     /* a work decomposition of the subject launches */
     struct Decomp {
@@ -268,6 +266,20 @@ struct ggdmc_session {
         int occ;
         bool wide;
     };
+    /* what a decomposition makes of the session's launches; computed before
+     * anything of the session changes, so that one that does not fit leaves
+     * the session as it is */
+    struct Layout {
+        Decomp c{};
+        std::vector<int4> items;      /* every launch's items, one launch after the other */
+        std::vector<int> list_n;
+        int kchain = 0, rmax = 1, cmax = 1, chain_batch = 1, tstage = 0;
+        bool tiled = false, overlap = false;
+        int ovl_stats_lds = 0;
+        size_t sweep_lds = 0, ovl_lds = 0;
+    };
+    Layout layout(Decomp c) const;
+    void use(const Layout &l);
     /* every iteration of every run is a plain crossover (the sampling phase):
      * no migration, blocked sweep, hyper-only run, trial tile or trace */
     bool lean() const {
@@ -695,53 +707,46 @@ void ggdmc_session::default_decomp() {
     if (cfg.chains_per_item < 0) {
         require(cfg.trials_per_tile == 0, "one item per subject needs trials_per_tile = 0");
         require(!one, "one item per subject already covers every group in one launch");
-        set_decomp(true, 0, 0);
+        use(layout({true, 0, 0, false, 1, false, 3, false}));
     } else if (cfg.chains_per_item > 0 || cfg.trials_per_tile > 0) {
-        set_decomp(false, cfg.chains_per_item, cfg.trials_per_tile, one, ipl_cfg, span_cfg, occ_cfg);
+        use(layout({false, cfg.chains_per_item, cfg.trials_per_tile, one, ipl_cfg, span_cfg, occ_cfg, false}));
     } else {
         int k = ngmax;
         while (k > 1 && (int64_t)d.S * ((ngmax + k - 1) / k) < 1024) k = (k + 1) / 2;
-        set_decomp(false, k, 0, one, ipl_cfg, span_cfg, occ_cfg);
+        use(layout({false, k, 0, one, ipl_cfg, span_cfg, occ_cfg, false}));
     }
 }
 
-/* Builds the item lists of the subject launches: per chain group, every
- * subject's chain ranges of k_new chains x trial tiles of tpt_new trials
- * (rounded up to a multiple of kChunk; 0 = whole subject); or, fused, one
- * item per subject that sweeps every group in one launch. Sizes the LDS. */
-void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chained_new, int ipl_new,
-                               bool span_new, int occ_new, bool wide_new) {
-    if (tpt_new > 0) tpt_new = ((tpt_new + kChunk - 1) / kChunk) * kChunk;
-    require(!fused_new || tpt_new == 0, "one item per subject needs whole subjects");
-    require(!(fused_new && chained_new), "one item per subject already covers every group");
-    require(!chained_new || nsweep_sub == 1, "every group in one launch needs unblocked subject sweeps");
-    require(ipl_new == 1 || chained_new, "several iterations per launch need every group in one launch");
-    require(!span_new || (chained_new && tpt_new == 0),
+/* The item lists of the subject launches: per chain group, every subject's
+ * chain ranges of c.k chains x trial tiles of c.tpt trials (rounded up to a
+ * multiple of kChunk; 0 = whole subject); or, fused, one item per subject that
+ * sweeps every group in one launch; and their LDS. Throws (GGDMC_EINVAL) where
+ * the decomposition does not fit this batch. */
+ggdmc_session::Layout ggdmc_session::layout(Decomp c) const {
+    if (c.tpt > 0) c.tpt = ((c.tpt + kChunk - 1) / kChunk) * kChunk;
+    require(!c.fused || c.tpt == 0, "one item per subject needs whole subjects");
+    require(!(c.fused && c.chained), "one item per subject already covers every group");
+    require(!c.chained || nsweep_sub == 1, "every group in one launch needs unblocked subject sweeps");
+    require(c.ipl == 1 || c.chained, "several iterations per launch need every group in one launch");
+    require(!c.span || (c.chained && c.tpt == 0),
             "items spanning every group need every group in one launch and whole subjects");
     const int n = d.nchain, G = d.G;
     const int ngmax = (n + G - 1) / G;
-    fused = fused_new;
-    chained = chained_new;
-    ipl = ipl_new;
-    span = span_new;
-    occ = ipl_new > 1 ? occ_new : 3;
-    wide = wide_new && ipl_new > 1;
-    tiled = false;
-    tpt = tpt_new;
-    d.tpt = tpt;
-    kchain = fused ? ngmax : std::min(k_new > 0 ? k_new : ngmax, ngmax);
-    lists.clear();
-    list_n.clear();
+    if (c.ipl == 1) {
+        c.occ = 3;
+        c.wide = false;
+    }
+    Layout l;
+    l.c = c;
+    l.kchain = c.fused ? ngmax : std::min(c.k > 0 ? c.k : ngmax, ngmax);
     int64_t max_chunks_item = 1;
-    const int nl = (fused || span) ? 1 : G;
-    std::vector<int4> all_items;   /* every group's items, in group order */
-    rmax = 1;
+    const int nl = (c.fused || c.span) ? 1 : G;
     /* XCD-aware order: workgroup w runs on XCD w % 8, so the items of subject
      * x go to workgroups w = x (mod 8) where possible, and share that XCD's
      * L2 for the subject's trials and state. The population workgroups come
      * first in a launch when the population step runs inside it. */
-    const bool phi_in = d.n_phi > 0 && d.S > 0 && !fused && nsweep_sub == 1;
-    int64_t wg_base = phi_in && chained ? (int64_t)d.n_phi * n : 0;
+    const bool phi_in = d.n_phi > 0 && d.S > 0 && !c.fused && nsweep_sub == 1;
+    int64_t wg_base = phi_in && c.chained ? (int64_t)d.n_phi * n : 0;
     auto xcd_order = [&](std::vector<int4> &v, int64_t base) {
         std::vector<std::vector<int4>> b(kXcd);
         for (const int4 &it : v) b[it.x % kXcd].push_back(it);
@@ -752,94 +757,66 @@ void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chai
             const int want = (int)((base + (int64_t)p) % kXcd);
             int pick = -1;
             for (int dx = 0; dx < kXcd && pick < 0; ++dx) {
-                const int c = (want + dx) % kXcd;
-                if (pos[c] < b[c].size()) pick = c;
+                const int q = (want + dx) % kXcd;
+                if (pos[q] < b[q].size()) pick = q;
             }
             out.push_back(b[pick][pos[pick]++]);
         }
         v.swap(out);
     };
     for (int g = 0; g < nl; ++g) {
-        const int ng = (fused || span) ? ngmax : (((g + 1) * n) / G - (g * n) / G);
-        const int nch = fused ? 1 : (ng + kchain - 1) / kchain;
+        const int ng = (c.fused || c.span) ? ngmax : (((g + 1) * n) / G - (g * n) / G);
+        const int nch = c.fused ? 1 : (ng + l.kchain - 1) / l.kchain;
         std::vector<int4> items;
         for (int x = 0; x < d.S; ++x) {
             const int64_t ntr = subj_ntr[x];
-            const int64_t nt = (tpt == 0 || ntr <= tpt) ? 1 : (ntr + tpt - 1) / tpt;
+            const int64_t nt = (c.tpt == 0 || ntr <= c.tpt) ? 1 : (ntr + c.tpt - 1) / c.tpt;
             require(nt <= 65535, "trials_per_tile too small for a subject's trial count");
-            tiled = tiled || nt > 1;
+            l.tiled = l.tiled || nt > 1;
             require((int64_t)nch * nt < (int64_t)1 << 30, "too many work items per subject");
             for (int ch = 0; ch < nch; ++ch) {
-                const int c0 = ch * kchain;
-                const int c1 = (fused || ch == nch - 1) ? kAllChains : c0 + kchain;
+                const int c0 = ch * l.kchain;
+                const int c1 = (c.fused || ch == nch - 1) ? kAllChains : c0 + l.kchain;
                 for (int64_t t = 0; t < nt; ++t)
                     items.push_back(make_int4(x, (c0 << 16) | c1, ((int)t << 16) | (int)nt, (g << 16) | ch));
             }
             max_chunks_item = std::max<int64_t>(max_chunks_item,
-                                                nt == 1 ? (ntr + kChunk - 1) / kChunk : tpt / kChunk);
+                                                nt == 1 ? (ntr + kChunk - 1) / kChunk : c.tpt / kChunk);
         }
-        rmax = std::max(rmax, nch);
-        require(!span || span_fits(nch), "too many chain ranges per subject for items spanning every group");
-        if (chained) {
-            xcd_order(items, wg_base);
-            wg_base += (int64_t)items.size();
-            all_items.insert(all_items.end(), items.begin(), items.end());
-            continue;
-        }
-        xcd_order(items, phi_in ? (int64_t)d.n_phi * ng : 0);
-        all_items.insert(all_items.end(), items.begin(), items.end());
-        list_n.push_back((int)items.size());
+        l.rmax = std::max(l.rmax, nch);
+        require(!c.span || span_fits(nch), "too many chain ranges per subject for items spanning every group");
+        xcd_order(items, c.chained ? wg_base : (phi_in ? (int64_t)d.n_phi * ng : 0));
+        l.items.insert(l.items.end(), items.begin(), items.end());
+        if (c.chained) wg_base += (int64_t)items.size();
+        else l.list_n.push_back((int)items.size());
     }
-    require(all_items.size() < ((size_t)1 << 31), "too many work items");
-    if (chained) list_n.push_back((int)all_items.size());
-    if (all_items.size() > list_cap) {
-        list_mem = pool.alloc<int4>(all_items.size());
-        list_cap = all_items.size();
-    }
-    if (!all_items.empty()) {
-        /* launches still running may read the lists: stream order, and the
-         * host vector lives until the copy is done */
-        HIPCHECK(hipMemcpyAsync(list_mem, all_items.data(), sizeof(int4) * all_items.size(), hipMemcpyHostToDevice,
-                                stream));
-        HIPCHECK(hipStreamSynchronize(stream));
-    }
-    size_t first = 0;
-    for (const int m : list_n) {
-        lists.push_back(list_mem + first);
-        first += (size_t)m;
-    }
-    {
-        const size_t nf = (size_t)std::max(d.S, 1) * G * rmax;
-        HIPCHECK(hipMemsetAsync(d.item_ready, 0, sizeof(uint32_t) * nf, stream));
-        HIPCHECK(hipMemsetAsync(d.item_staged, 0, sizeof(uint32_t) * nf, stream));
-        HIPCHECK(hipMemsetAsync(d.tile_ctr, 0, sizeof(uint32_t) * nf, stream));
-    }
+    require(l.items.size() < ((size_t)1 << 31), "too many work items");
+    if (c.chained) l.list_n.push_back((int)l.items.size());
     /* LDS: accumulator constants of chain_batch chains and cmax chunk sums
      * per chain at once, within 48 KB when possible */
-    kmax = kchain;
-    cmax = (int)std::min<int64_t>(max_chunks_item, std::max(1, 4096 / kmax));
-    chain_batch = kmax;
+    const int kmax = l.kchain;
+    l.cmax = (int)std::min<int64_t>(max_chunks_item, std::max(1, 4096 / kmax));
+    l.chain_batch = kmax;
     const int per_chain = d.n_cond * d.n_acc;
     /* the item's trials in LDS when they fit in 24 KB */
     int64_t max_item_trials = 0;
     for (int x = 0; x < d.S; ++x)
         max_item_trials = std::max<int64_t>(max_item_trials,
-                                            tpt == 0 ? subj_ntr[x] : std::min<int64_t>(tpt, subj_ntr[x]));
-    tstage = max_item_trials * 10 <= 24 * 1024 ? (int)max_item_trials : 0;
+                                            c.tpt == 0 ? subj_ntr[x] : std::min<int64_t>(c.tpt, subj_ntr[x]));
+    l.tstage = max_item_trials * 10 <= 24 * 1024 ? (int)max_item_trials : 0;
     auto bytes = [&]() {
-        return ggdmc_internal_sweep_lds(n, d.P, kmax, per_chain, chain_batch, cmax, tstage);
+        return ggdmc_internal_sweep_lds(n, d.P, kmax, per_chain, l.chain_batch, l.cmax, l.tstage);
     };
     const size_t soft = 48 * 1024, limit = (size_t)device_lds_limit();
-    while (chain_batch > 1 && bytes() > soft) --chain_batch;
-    while (cmax > 1 && bytes() > soft) cmax = (cmax + 1) / 2;
-    if (bytes() > soft) tstage = 0;
-    sweep_lds = bytes();
-    require(sweep_lds <= limit, "design too large for LDS (chains x parameters)");
+    while (l.chain_batch > 1 && bytes() > soft) --l.chain_batch;
+    while (l.cmax > 1 && bytes() > soft) l.cmax = (l.cmax + 1) / 2;
+    if (bytes() > soft) l.tstage = 0;
+    l.sweep_lds = bytes();
+    require(l.sweep_lds <= limit, "design too large for LDS (chains x parameters)");
     /* the population step of each chain group runs in that group's subject
      * launch (not with one item per subject over every group, nor with
      * blocked subject sweeps: those keep the population kernel) */
-    overlap = false;
-    if (d.n_phi > 0 && d.S > 0 && !fused && nsweep_sub == 1) {
+    if (phi_in) {
         const int max_sub = (int)(d.bstats_stride / 4 / ((int64_t)n * d.P)) * kStatBlock;
         /* the whole-run population step (its LDS holds the whole population
          * state) runs in these launches only for hyper-only runs, blocked
@@ -847,14 +824,59 @@ void ggdmc_session::set_decomp(bool fused_new, int k_new, int tpt_new, bool chai
          * workgroup needs only the per-chain step's or an item's LDS */
         bool whole_run = d.blocked_pop != 0 || d.pop_mig > 0.0;
         for (const ggdmc_job &j : jobs) whole_run = whole_run || j.kind == GGDMC_KIND_HYPER;
-        ovl_stats_lds = ggdmc_internal_phi_lds(n, d.P, G, 1) <= limit ? 1 : 0;
-        ovl_lds = std::max({sweep_lds, whole_run ? ggdmc_internal_phi_lds(n, d.P, G, ovl_stats_lds) : (size_t)0,
-                            ggdmc_internal_phi_chain_lds(d.P, max_sub)});
-        overlap = ovl_lds <= limit;
+        l.ovl_stats_lds = ggdmc_internal_phi_lds(n, d.P, G, 1) <= limit ? 1 : 0;
+        l.ovl_lds = std::max({l.sweep_lds, whole_run ? ggdmc_internal_phi_lds(n, d.P, G, l.ovl_stats_lds) : (size_t)0,
+                              ggdmc_internal_phi_chain_lds(d.P, max_sub)});
+        l.overlap = l.ovl_lds <= limit;
     }
-    require(ipl == 1 || d.n_phi == 0 || overlap,
+    require(c.ipl == 1 || d.n_phi == 0 || l.overlap,
             "several iterations per launch need the population step inside the subject launch");
+    return l;
+}
+
+/* The launches from here on follow l. */
+void ggdmc_session::use(const Layout &l) {
     drop_graph();
+    if (l.items.size() > list_cap) {
+        list_mem = pool.alloc<int4>(l.items.size());
+        list_cap = l.items.size();
+    }
+    if (!l.items.empty()) {
+        /* launches still running may read the lists: stream order, and the
+         * host vector lives until the copy is done */
+        HIPCHECK(hipMemcpyAsync(list_mem, l.items.data(), sizeof(int4) * l.items.size(), hipMemcpyHostToDevice,
+                                stream));
+        HIPCHECK(hipStreamSynchronize(stream));
+    }
+    lists.clear();
+    size_t first = 0;
+    for (const int m : l.list_n) {
+        lists.push_back(list_mem + first);
+        first += (size_t)m;
+    }
+    list_n = l.list_n;
+    fused = l.c.fused;
+    chained = l.c.chained;
+    ipl = l.c.ipl;
+    span = l.c.span;
+    occ = l.c.occ;
+    wide = l.c.wide;
+    tiled = l.tiled;
+    tpt = l.c.tpt;
+    d.tpt = tpt;
+    kchain = kmax = l.kchain;
+    rmax = l.rmax;
+    cmax = l.cmax;
+    chain_batch = l.chain_batch;
+    tstage = l.tstage;
+    sweep_lds = l.sweep_lds;
+    overlap = l.overlap;
+    ovl_stats_lds = l.ovl_stats_lds;
+    ovl_lds = l.ovl_lds;
+    const size_t nf = (size_t)std::max(d.S, 1) * d.G * rmax;
+    HIPCHECK(hipMemsetAsync(d.item_ready, 0, sizeof(uint32_t) * nf, stream));
+    HIPCHECK(hipMemsetAsync(d.item_staged, 0, sizeof(uint32_t) * nf, stream));
+    HIPCHECK(hipMemsetAsync(d.tile_ctr, 0, sizeof(uint32_t) * nf, stream));
 }
 
 /* One iteration's launches: the population step of the iteration (from the
@@ -1000,13 +1022,16 @@ void ggdmc_session::run_plain(uint32_t n_iter) {
     }
 }
 
+/* Takes decomposition c if it fits; the session is unchanged if not. */
 bool ggdmc_session::try_decomp(const Decomp &c) {
+    Layout l;
     try {
-        set_decomp(c.fused, c.k, c.tpt, c.chained, c.ipl, c.span, c.occ, c.wide);
-    } catch (const Error &) {
-        if (c.ipl == 1) throw;
-        return false;   /* no population step inside the launch for this design */
+        l = layout(c);
+    } catch (const Error &e) {
+        if (e.code != GGDMC_EINVAL) throw;
+        return false;
     }
+    use(l);
     return true;
 }
 
@@ -1122,8 +1147,9 @@ void ggdmc_session::run_whole() {
         return;
     }
     const std::vector<Decomp> cands = candidates();
+    /* the first that fits; none: the default of build() stays */
     size_t pick = 0;
-    while (!try_decomp(cands[pick])) ++pick;
+    while (pick < cands.size() && !try_decomp(cands[pick])) ++pick;
     auto run = [&](uint32_t cnt) {
         run_batched(cnt);
         left -= cnt;
@@ -1140,7 +1166,7 @@ void ggdmc_session::run_whole() {
         HIPCHECK(hipEventElapsedTime(&ms, e0.get(), e1.get()));
         return ms / (float)cnt;
     };
-    if (left >= 6 * unit()) {
+    if (pick < cands.size() && left >= 6 * unit()) {
         const uint32_t total = left;
         size_t now = pick;
         run(unit());   /* the first launch of a process loads the code */
@@ -1253,7 +1279,7 @@ void ggdmc_session::autotune() {
         }
     }
     next_iter = it0;
-    try_decomp(pick);
+    if (best < 1e30f) try_decomp(pick);   /* none fits: the default of build() stays */
 }
 
 static int fail(const std::exception &e) {

@@ -1,0 +1,59 @@
+"""Work decompositions at the edges of what fits: a candidate that does not fit
+is passed over, and no decomposition changes a bit."""
+import numpy as np
+import pytest
+
+from ggdmc_amd import priors
+from ggdmc_amd.model import build_model
+from ggdmc_amd.simulate import simulate_subject
+
+pytestmark = pytest.mark.gpu
+
+
+def _thresholds_job(gpu, levels, nchain, per_level, seed=3):
+    """Model and single-subject job with one threshold per stimulus: levels + 4
+    parameters, levels x 2 condition x accumulator pairs."""
+    stim = ["s%d" % i for i in range(levels)]
+    m = build_model(p_map={"A": ["1"], "B": ["S"], "t0": ["1"], "mean_v": ["M"], "sd_v": ["1"], "st0": ["1"]},
+                    match_map={"M": {s: ("r1", "r2")[i % 2] for i, s in enumerate(stim)}},
+                    factors={"S": stim}, constants={"st0": 0.0, "sd_v": 1.0}, accumulators=["r1", "r2"])
+    rng = np.random.default_rng(seed)
+    x = np.array([{"A": 0.4, "t0": 0.1, "mean_v.true": 3.0, "mean_v.false": 1.0}.get(p, 1.2) for p in m.pnames])
+    data = simulate_subject(m, x, per_level, rng)
+    prior = gpu.PriorSpec.uniform(m.npar, 0.0, 10.0, m.pnames)
+    th = x[:, None] * np.exp(rng.normal(0, 0.03, (m.npar, nchain)))
+    lp = np.array([priors.sumlogprior(prior, th[:, c]) for c in range(nchain)])
+    ll = gpu.loglike(m, data, th.T.copy(), gpu.FP64_PLAIN)
+    return m, gpu.JobSpec(gpu.KIND_SUBJECT, seed, prior, start=(th, lp, ll), subject=data)
+
+
+def _session(gpu, cfg, m, jobs):
+    s = gpu.Session(gpu.make_config(**cfg), m, jobs)
+    s.advance(s.total_iters)
+    res = s.download()
+    s.close()
+    return res
+
+
+def _same(a, b):
+    for x, y in zip(a, b):
+        for p, q in zip(x["subjects"], y["subjects"]):
+            assert np.array_equal(p.theta, q.theta)
+            assert np.array_equal(p.summed_log_prior, q.summed_log_prior)
+            assert np.array_equal(p.log_likelihoods, q.log_likelihoods)
+
+
+@pytest.mark.parametrize("precision", ["MIXED_BATCHED", "FP64_BATCHED"])
+def test_a_candidate_too_large_for_lds_is_passed_over(gpu, precision):
+    # 30 parameters, 90 chains: an item of a whole chain group takes 97 KB of
+    # LDS, one chain 26 KB; blocked sweeps rank the former among the candidates
+    m, job = _thresholds_job(gpu, 26, 90, 2)
+    assert m.npar == 30
+    cfg = dict(nmc=67, nchain=90, is_pblocked=True, precision=getattr(gpu, precision))
+    got = gpu.run_batch(gpu.make_config(**cfg), m, [job])
+    s = gpu.Session(gpu.make_config(**cfg), m, [job])
+    assert s.decomposition()[0] != -1
+    s.advance(s.total_iters)
+    _same(got, s.download())
+    s.close()
+    _same(got, _session(gpu, dict(cfg, launch_mode=1, chains_per_item=2), m, [job]))
