@@ -28,15 +28,13 @@
 #include <cstdint>
 
 #include "../../include/ggdmc_hip.h"
+#include "work_split.h"
 
 namespace ggdmc {
 
-constexpr int kBlock = 256;        /* threads per workgroup of the sweep kernels */
-constexpr int kWideBlock = 512;    /* ... of their build for launches of few items */
+constexpr int kWideBlock = 512;    /* threads of the sweep kernels' build for launches of few items */
 constexpr int kPhiBlock = 512;     /* threads per workgroup of the population kernel */
-constexpr int kWaves = kBlock / 64;
 constexpr int kMaxChains = 256;    /* chains per run */
-constexpr int kChunk = 128;        /* trials per canonical chunk sum */
 constexpr int kStatBlock = 32;     /* subjects per block of the population statistics */
 constexpr uint32_t kHyperItersPerLaunch = 256; /* iterations per launch of hyper-only runs */
 constexpr int kItersPerLaunch = 32; /* iterations per subject launch in launch mode 3 */

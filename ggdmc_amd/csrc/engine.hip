@@ -1074,21 +1074,20 @@ std::vector<ggdmc_session::Decomp> ggdmc_session::candidates() const {
     }
     const int k = ks[i];
     std::vector<Decomp> out;
+    /* launches whose workgroups wait for each other: only while the waits fit */
+    auto can_wait = [&](int kk) {
+        return waits_fit(max_ntr, d.n_acc, mode == GGDMC_FP64_BATCHED, d.G, std::min(kk, ng),
+                         d.sub_mig > 0.0 ? d.nchain : 0);
+    };
     auto add = [&](const Decomp &c) {
+        if (c.chained && !can_wait(c.k)) return;
         for (const Decomp &o : out)
             if (o.fused == c.fused && o.k == c.k && o.tpt == c.tpt && o.chained == c.chained && o.ipl == c.ipl &&
                 o.span == c.span && o.occ == c.occ && o.wide == c.wide)
                 return;
         out.push_back(c);
     };
-    /* several iterations per launch wait for each other's items a bounded time
-     * (kSpinLimit polls, about 0.4 s): an item's likelihoods, or a migration
-     * ring's, must stay far below it. A chunk of a chain takes a wave about 4 us
-     * with 2 accumulators, three times that in FP64. */
-    const double chunk_us = 2.0 * d.n_acc * (mode == GGDMC_FP64_BATCHED ? 3.0 : 1.0);
-    const double rounds = std::ceil((double)max_ntr / kChunk / kWaves);
-    const bool can_chain = nsweep_sub == 1 && cfg.launch_mode != 1 &&
-                           rounds * chunk_us * std::max(k, d.sub_mig > 0.0 ? d.nchain : 1) < 5e4;
+    const bool can_chain = nsweep_sub == 1 && cfg.launch_mode != 1 && can_wait(k);
     if (can_chain) {
         /* 8 waves per workgroup where every workgroup of two segments has a CU
          * to itself and 4 waves would take an item's chunks in several rounds

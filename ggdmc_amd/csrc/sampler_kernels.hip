@@ -1642,10 +1642,16 @@ constexpr uint32_t kSpinLimit = 1u << 18;
  * several iterations in a launch a flag may already hold a later one). */
 __device__ __forceinline__ bool reached(uint32_t v, uint32_t iter) { return (int32_t)(v - iter) >= 0; }
 
-/* One flag, by one thread. */
+/* One flag, by one thread. The bound counts from the flag's last advance: in a
+ * launch of several iterations a workgroup may be resident, and waiting, that
+ * many iterations before its turn. */
 __device__ __forceinline__ void wait_flag(const Dev &d, const uint32_t *flag, uint32_t iter) {
-    uint32_t spins = 0;
-    while (!reached(__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), iter)) {
+    uint32_t spins = 0, seen = iter;
+    for (;;) {
+        const uint32_t v = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (reached(v, iter)) break;
+        if (v != seen) spins = 0;
+        seen = v;
         /* after one failure every later wait gives up at once */
         if (++spins == kSpinLimit || __hip_atomic_load(d.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
             atomicOr(d.fault, 1u);

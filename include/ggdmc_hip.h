@@ -72,7 +72,9 @@ typedef struct {
                                also waits for its subject's previous iteration), 4 = as 3
                                with an item holding its chain range of every group (its
                                later groups wait for the earlier groups' items); never
-                               changes results */
+                               changes results. 2 to 4 are refused at run time (GGDMC_EHIP)
+                               where one iteration of a subject takes 0.4 s, the bound of a
+                               wait; 0 leaves them out from 50 ms */
     uint64_t iter_offset;   /* Philox iteration offset (restart continues a stream) */
     int32_t pop_debug;      /* de_input@pop_debug: record the population level's decisions */
     int32_t sub_debug;      /* de_input@sub_debug: record the decisions of single-subject and

@@ -4,6 +4,7 @@
 // without a GPU.
 #include "../../ggdmc_amd/csrc/fp64_math.h"
 #include "../../ggdmc_amd/csrc/lba_math.h"
+#include "../../ggdmc_amd/csrc/work_split.h"
 
 #include <cmath>
 #include <vector>
@@ -29,6 +30,15 @@ struct HostOps {
 } // namespace
 
 extern "C" {
+
+// The rule that keeps launches whose workgroups wait for each other to
+// iterations far below the bound of a wait.
+double host_iteration_us(int64_t ntrial, int n_acc, int fp64, int G, int k, int ring_chains) {
+    return ggdmc::iteration_us(ntrial, n_acc, fp64 != 0, G, k, ring_chains);
+}
+int host_waits_fit(int64_t ntrial, int n_acc, int fp64, int G, int k, int ring_chains) {
+    return ggdmc::waits_fit(ntrial, n_acc, fp64 != 0, G, k, ring_chains);
+}
 
 // x[i] / d[i] through the batched path's division from the reciprocal.
 void host_div_rn(const double *x, const double *d, int64_t n, double *out) {

@@ -3,6 +3,7 @@ is passed over, and no decomposition changes a bit."""
 import numpy as np
 import pytest
 
+import fixtures as fx
 from ggdmc_amd import priors
 from ggdmc_amd.model import build_model
 from ggdmc_amd.simulate import simulate_subject
@@ -57,3 +58,21 @@ def test_a_candidate_too_large_for_lds_is_passed_over(gpu, precision):
     _same(got, s.download())
     s.close()
     _same(got, _session(gpu, dict(cfg, launch_mode=1, chains_per_item=2), m, [job]))
+
+
+def test_a_launch_may_take_longer_than_the_bound_of_a_wait(gpu):
+    # 32 iterations of about 20 ms in one launch: its last segment's workgroup
+    # is resident, and waiting, from the start, and the bound of a wait (about
+    # 0.4 s) counts from the awaited subject's last iteration
+    fix = fx.load("lba_data6")
+    cells = [np.resize(fix.sub_data.rt[a:b], 60000 * (b - a) // len(fix.sub_data.rt))
+             for a, b in zip(fix.sub_data.cell_off[:-1], fix.sub_data.cell_off[1:])]
+    data = gpu.SubjectData.from_cells(cells)
+    rng = np.random.default_rng(2)
+    th = fx.truth_vector(fix)[:, None] * np.exp(rng.normal(0, 0.02, (fix.P, 39)))
+    lp = np.array([priors.sumlogprior(fix.sub_prior, th[:, c]) for c in range(39)])
+    job = gpu.JobSpec(gpu.KIND_SUBJECT, 11, fix.sub_prior, subject=data,
+                      start=(th, lp, gpu.loglike(fix.model, data, th.T.copy(), gpu.FP64_PLAIN)))
+    cfg = dict(nmc=34, nchain=39, sweep_groups=39, precision=gpu.FP64_BATCHED, chains_per_item=1)
+    _same(_session(gpu, dict(cfg, launch_mode=4), fix.model, [job]),
+          _session(gpu, dict(cfg, launch_mode=1), fix.model, [job]))
