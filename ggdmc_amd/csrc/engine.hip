@@ -304,6 +304,16 @@ struct ggdmc_session {
     void capture(int K);
     hipGraphExec_t make_graph(int K);
     void prepare_rest(uint32_t n_iter);
+    /* the caller's sample buffers, which the downloads write on the host */
+    void check_outs() const {
+        auto check = [](const ggdmc_samples &o) { require(o.theta && o.lp && o.ll, "sample buffer missing"); };
+        for (const ggdmc_job &j : jobs) {
+            if (j.kind != GGDMC_KIND_SUBJECT) check(*j.phi_out);
+            if (j.kind == GGDMC_KIND_HYPER) continue;
+            const int ns = j.kind == GGDMC_KIND_SUBJECT ? 1 : j.nsubject;
+            for (int k = 0; k < ns; ++k) check(j.subject_outs[k]);
+        }
+    }
     /* a subject workgroup gave up waiting for the population step */
     void check_fault() {
         uint32_t f = 0;
@@ -1473,6 +1483,7 @@ int ggdmc_session_profile(ggdmc_session *s, int32_t n_iter, double *subject_kern
 int ggdmc_session_download(ggdmc_session *s) {
     if (!s) return invalid("session is null");
     try {
+        s->check_outs();
         const size_t nmc = (size_t)s->cfg.nmc, n = (size_t)s->d.nchain, P = (size_t)s->d.P;
         HIPCHECK(hipStreamSynchronize(s->stream));
         /* the caller's buffers of every population state and subject, in the
@@ -1544,6 +1555,7 @@ int ggdmc_run_batch(const ggdmc_config *cfg, const ggdmc_model *model, const ggd
     int rc = GGDMC_OK;
     try {
         s->build(cfg, model, jobs, njobs);
+        s->check_outs();
         s->run_timed(0, true);
     } catch (const std::exception &e) {
         rc = fail(e);

@@ -202,7 +202,8 @@ int ggdmc_session_create(const ggdmc_config *cfg, const ggdmc_model *model,
 int ggdmc_session_advance(ggdmc_session *s, int32_t n_iter);
 /* Device time in ms of the last advance (HIP events on the session stream). */
 int ggdmc_session_elapsed_ms(ggdmc_session *s, float *ms);
-/* Copies every job's stored samples into its *_out buffers. */
+/* Copies every job's stored samples into its *_out buffers; a null buffer is
+ * refused (GGDMC_EINVAL). */
 int ggdmc_session_download(ggdmc_session *s);
 /* Average device time (ms) of the subject-level kernel over n_iter
  * iterations run launch by launch with events around each launch, and the
