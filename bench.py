@@ -94,7 +94,7 @@ def parse():
     ap.add_argument("--decomp", default="",
                     help="fixed work items 'k,t[,m[,w]]' (chains per item or -1, trials per item "
                          "or 0, launch mode 1 to 4 as make_config's launch_mode, waves per SIMD "
-                         "of the subject kernel 3 or 4) instead of autotuning")
+                         "of the subject kernel 2, 3 or 4) instead of autotuning")
     ap.add_argument("--calibrate-copy", action="store_true",
                     help="only run a 256 MiB device-to-device copy (counter calibration)")
     return ap.parse_args()

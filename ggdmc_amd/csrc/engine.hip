@@ -711,19 +711,21 @@ void ggdmc_session::default_decomp() {
     const bool one = cfg.launch_mode >= 2;
     const int ipl_cfg = cfg.launch_mode >= 3 ? kItersPerLaunch : 1;
     const bool span_cfg = cfg.launch_mode == 4;
-    require(cfg.waves_per_simd == 0 || cfg.waves_per_simd == 3 || cfg.waves_per_simd == 4,
-            "waves_per_simd must be 0, 3 or 4");
+    require(cfg.waves_per_simd == 0 || cfg.waves_per_simd == 3 || cfg.waves_per_simd == 4 ||
+                (cfg.waves_per_simd == 2 && cfg.launch_mode >= 3),
+            "waves_per_simd must be 0, 3 or 4, or 2 with launch mode 3 or 4");
     const int occ_cfg = cfg.waves_per_simd == 4 && ipl_cfg > 1 ? 4 : 3;
+    const bool wide_cfg = cfg.waves_per_simd == 2;
     if (cfg.chains_per_item < 0) {
         require(cfg.trials_per_tile == 0, "one item per subject needs trials_per_tile = 0");
         require(!one, "one item per subject already covers every group in one launch");
         use(layout({true, 0, 0, false, 1, false, 3, false}));
     } else if (cfg.chains_per_item > 0 || cfg.trials_per_tile > 0) {
-        use(layout({false, cfg.chains_per_item, cfg.trials_per_tile, one, ipl_cfg, span_cfg, occ_cfg, false}));
+        use(layout({false, cfg.chains_per_item, cfg.trials_per_tile, one, ipl_cfg, span_cfg, occ_cfg, wide_cfg}));
     } else {
         int k = ngmax;
         while (k > 1 && (int64_t)d.S * ((ngmax + k - 1) / k) < 1024) k = (k + 1) / 2;
-        use(layout({false, k, 0, one, ipl_cfg, span_cfg, occ_cfg, false}));
+        use(layout({false, k, 0, one, ipl_cfg, span_cfg, occ_cfg, wide_cfg}));
     }
 }
 
@@ -1410,7 +1412,7 @@ int ggdmc_session_elapsed_ms(ggdmc_session *s, float *ms) {
 
 int ggdmc_session_waves_per_simd(ggdmc_session *s, int32_t *waves_per_simd) {
     if (!s || !waves_per_simd) return invalid("session / waves_per_simd is null");
-    *waves_per_simd = s->occ;
+    *waves_per_simd = s->wide ? 2 : s->occ;
     return GGDMC_OK;
 }
 

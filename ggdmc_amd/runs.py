@@ -175,10 +175,10 @@ def make_config(nmc, nchain, thin=1, pop_migration_prob=0.0, sub_migration_prob=
     library autotune the work split; launch_mode 1 = a subject launch per chain
     group, 2 = one for every group, 3 = one for every group and 32 iterations,
     4 = as 3 with an item holding its chain range of every group.
-    waves_per_simd (0 = autotuned, 3 or 4) picks the build of the subject kernel
-    for launch modes 3 and 4. None of them changes a result bit. pop_debug /
-    sub_debug record the decisions of the population level / of the subjects
-    (Session.trace)."""
+    waves_per_simd (0 = autotuned, 3 or 4, or 2: 8 waves per workgroup, with
+    launch_mode 3 or 4 given) picks the build of the subject kernel for launch
+    modes 3 and 4. None of them changes a result bit. pop_debug / sub_debug record
+    the decisions of the population level / of the subjects (Session.trace)."""
     return _lib.Config(int(nmc), int(thin), int(nchain), float(pop_migration_prob),
                        float(sub_migration_prob), float(gamma_precursor), float(rp),
                        int(bool(is_hblocked)), int(bool(is_pblocked)), int(precision),
@@ -338,7 +338,8 @@ class Session:
         return k.value, t.value, m.value, lm.value
 
     def waves_per_simd(self):
-        """Waves per SIMD the subject kernel of this session was built for (3 or 4)."""
+        """Waves per SIMD the subject kernel of this session was built for (3 or 4,
+        or 2: 8 waves per workgroup), as make_config's waves_per_simd."""
         w = C.c_int32()
         check(_lib.lib().ggdmc_session_waves_per_simd(self.h, C.byref(w)))
         return w.value

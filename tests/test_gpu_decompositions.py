@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import fixtures as fx
-from ggdmc_amd import priors
+from ggdmc_amd import priors, workloads
 from ggdmc_amd.model import build_model
 from ggdmc_amd.simulate import simulate_subject
 
@@ -76,3 +76,36 @@ def test_a_launch_may_take_longer_than_the_bound_of_a_wait(gpu):
     cfg = dict(nmc=34, nchain=39, sweep_groups=39, precision=gpu.FP64_BATCHED, chains_per_item=1)
     _same(_session(gpu, dict(cfg, launch_mode=4), fix.model, [job]),
           _session(gpu, dict(cfg, launch_mode=1), fix.model, [job]))
+
+
+@pytest.mark.parametrize("precision", ["MIXED_BATCHED", "FP64_BATCHED"])
+@pytest.mark.parametrize("mig", [0.0, 0.2])     # the build for plain crossovers, the general one
+def test_the_eight_wave_build_can_be_asked_for(gpu, mig, precision):
+    # one subject's fit: the library takes this build by itself, and the
+    # decomposition and build a session reports are the ones that give it again
+    fix = fx.load("lba_data6")
+    th, lp, ll = fx.near_start(fix, 39, seed=8, scale=0.02)
+    job = gpu.JobSpec(gpu.KIND_SUBJECT, 3, fix.sub_prior, start=(th, lp, ll), subject=fix.sub_data)
+    cfg = dict(nmc=40, nchain=39, sub_migration_prob=mig, precision=getattr(gpu, precision))
+    want = _session(gpu, dict(cfg, launch_mode=1, chains_per_item=1), fix.model, [job])
+    for k, tpt, mode, w in ((1, 0, 4, 2), (1, 0, 3, 2), (20, 0, 4, 2), (4, 128, 3, 2)):
+        s = gpu.Session(gpu.make_config(**cfg, chains_per_item=k, trials_per_tile=tpt, launch_mode=mode,
+                                        waves_per_simd=w), fix.model, [job])
+        assert s.decomposition()[:2] == (k, tpt) and s.decomposition()[3] == mode
+        assert s.waves_per_simd() == 2
+        s.advance(s.total_iters)
+        _same(want, s.download())
+        s.close()
+    with pytest.raises(gpu.GgdmcError, match="waves_per_simd"):
+        gpu.Session(gpu.make_config(**cfg, chains_per_item=1, launch_mode=2, waves_per_simd=2), fix.model, [job])
+
+
+def test_the_eight_wave_build_in_a_hierarchical_run(gpu):
+    w = workloads.make("c3", scale=0.1)
+    for kw in ({}, {"pop_migration_prob": 0.2, "sub_migration_prob": 0.2}, {"is_hblocked": True}):
+        cfg = dict(nmc=35, nchain=w.nchain, **kw)
+        want = _session(gpu, dict(cfg, launch_mode=1, chains_per_item=4), w.model, w.jobs)
+        got = _session(gpu, dict(cfg, launch_mode=4, chains_per_item=1, waves_per_simd=2), w.model, w.jobs)
+        _same(want, got)
+        assert np.array_equal(want[0]["phi"].theta, got[0]["phi"].theta)
+        assert np.array_equal(want[0]["phi"].log_likelihoods, got[0]["phi"].log_likelihoods)
