@@ -1627,45 +1627,19 @@ int ggdmc_loglike_noalloc(const ggdmc_model *model, const ggdmc_subject *data, c
 
 } // extern "C"
 
-/* The split of a likelihood call. Per workgroup the constants take about 4 us
- * whatever k, a chunk of one vector about 3 us of one wave; about 3 workgroups
- * of 4 waves are resident on a CU. Times of whole calls, about 50 us of each
- * outside the kernel:
- *   - few vectors and chunks (at most 8 chunks per CU): one workgroup of 8
- *     waves per vector and 8 chunks, one chunk a wave, so that the call is one
- *     set-up and one chunk long (1 x 768: 55.5 us, 4 waves in two rounds 60.6);
- *   - two vectors per CU or more: 4 waves and whole vectors, k of them together
- *     while a wave has less than 6 chunks and 3.5 workgroups per CU remain, for
- *     one set-up per k (8190 x 768: k = 1 176 us, 2 159, 4 153; 2000 x 768: 84,
- *     80, 82; 624 x 768: 65, 66, 69; 1000 x 2047 of 4 accumulators: 93, 99,
- *     114);
- *   - a long subject under few vectors: 4 waves and 16 chunks (4 a wave), fewer
- *     while that leaves less than 3 workgroups per CU (33 x 100608 of 4
- *     accumulators: 4 chunks 197 us, 8 to 24 181, 48 198, one workgroup per
- *     vector 804; 4 x 100608: 4 and 8 chunks 132, 16 138, 32 150).
- * The first stages its trials in LDS with the set-up's loads; the others read
- * them from L2 as they go (staged: 1000 x 2047 93 us instead of 90).
- * may_split false: no chunk sums in memory, whole vectors only. */
+/* The split of a likelihood call (loglike_shape) and its LDS. may_split false:
+ * no chunk sums in memory, whole vectors only. */
 static LoglikeSplit loglike_split(int n, int64_t ntrial, int per_chain, int P, bool may_split) {
     LoglikeSplit sp{};
     sp.n = n;
     sp.ntrial = ntrial;
     sp.nj = (int)((ntrial + kChunk - 1) / kChunk);
     const int nj = std::max(sp.nj, 1);
-    const int64_t cus = std::max(device_cus(), 1);
-    sp.k = 1;
-    sp.threads = 256;
-    sp.jper = nj;
-    if (may_split && (int64_t)n * ((nj + 7) / 8) <= cus) {
-        sp.jper = std::min(nj, 8);
-        sp.threads = nj > 4 ? 512 : 256;
-        sp.tstage = (int)std::min<int64_t>((int64_t)sp.jper * kChunk, ntrial);
-    } else if (n >= 2 * cus || !may_split) {
-        while (sp.k < 4 && sp.k * nj < 24 && n / (sp.k + 1) >= 7 * cus / 2) ++sp.k;
-    } else {
-        sp.jper = std::min(nj, 16);
-        while (sp.jper > 4 && (int64_t)n * ((nj + sp.jper - 1) / sp.jper) < 3 * cus) sp.jper -= 4;
-    }
+    const LoglikeShape sh = loglike_shape(n, nj, std::max(device_cus(), 1), may_split);
+    sp.k = sh.k;
+    sp.threads = sh.threads;
+    sp.jper = sh.jper;
+    if (sh.stage) sp.tstage = (int)std::min<int64_t>((int64_t)sp.jper * kChunk, ntrial);
     sp.nsplit = (nj + sp.jper - 1) / sp.jper;
     sp.cmax = std::min(sp.jper, sp.nsplit > 1 ? 256 : 1024 / sp.k);
     if (sp.nsplit > 1) sp.cmax = std::max(sp.cmax, std::min(nj, 256));

@@ -40,6 +40,15 @@ int host_waits_fit(int64_t ntrial, int n_acc, int fp64, int G, int k, int ring_c
     return ggdmc::waits_fit(ntrial, n_acc, fp64 != 0, G, k, ring_chains);
 }
 
+// The split of a likelihood call: out = {vectors, threads, chunks per workgroup, staged}.
+void host_loglike_shape(int64_t n, int nj, int64_t cus, int may_split, int *out) {
+    const ggdmc::LoglikeShape s = ggdmc::loglike_shape(n, nj, cus, may_split != 0);
+    out[0] = s.k;
+    out[1] = s.threads;
+    out[2] = s.jper;
+    out[3] = s.stage;
+}
+
 // x[i] / d[i] through the batched path's division from the reciprocal.
 void host_div_rn(const double *x, const double *d, int64_t n, double *out) {
     for (int64_t i = 0; i < n; ++i) {

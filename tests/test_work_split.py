@@ -37,3 +37,37 @@ def test_waits_are_bounded_by_one_iteration(case, fits):
     want = rounds * 2.0 * acc * (3 if fp64 else 1) * max(G * k, ring)
     assert L.host_iteration_us(*case) == want
     assert fits == (want < 50_000)
+
+
+def _shape(n, nj, cus=256, may_split=True):
+    out = (C.c_int * 4)()
+    L = _lib()
+    L.host_loglike_shape.argtypes = [C.c_int64, C.c_int, C.c_int64, C.c_int, C.POINTER(C.c_int)]
+    L.host_loglike_shape(n, nj, cus, int(may_split), out)
+    return list(out)
+
+
+@pytest.mark.parametrize("n", [1, 3, 33, 64, 130, 200, 256, 257, 400, 511, 512, 520, 8190])
+def test_a_split_vector_gives_every_wave_a_chunk(n):
+    # off-multiple chunk counts too: 9 or 13 chunks had been split into
+    # workgroups of one chunk with three idle waves, 17 into 16 and 1
+    for nj in list(range(1, 120)) + [786, 5000]:
+        k, threads, jper, stage = _shape(n, nj)
+        parts = -(-nj // jper)
+        if parts > 1:
+            assert k == 1
+            if stage:
+                assert (threads, jper) == (512, 8) and n * -(-nj // 8) <= 256
+            else:
+                assert threads == 256 and n < 512 and nj >= 7
+                assert 3 <= jper <= 16
+                assert jper == -(-nj // parts)      # evenly
+        # may not split: whole vectors
+        assert -(-nj // _shape(n, nj, may_split=False)[2]) == 1
+
+
+@pytest.mark.parametrize("n,nj,jper", [(200, 9, 3), (200, 13, 4), (400, 5, 5), (400, 6, 6), (400, 8, 4),
+                                       (400, 10, 5), (500, 17, 9), (300, 17, 6), (33, 786, 16), (4, 786, 4),
+                                       (511, 33, 11)])
+def test_chunks_per_workgroup(n, nj, jper):
+    assert _shape(n, nj)[2] == jper
