@@ -792,8 +792,14 @@ ggdmc_session::Layout ggdmc_session::layout(Decomp c) const {
                 for (int64_t t = 0; t < nt; ++t)
                     items.push_back(make_int4(x, (c0 << 16) | c1, ((int)t << 16) | (int)nt, (g << 16) | ch));
             }
-            max_chunks_item = std::max<int64_t>(max_chunks_item,
-                                                nt == 1 ? (ntr + kChunk - 1) / kChunk : c.tpt / kChunk);
+            /* a migration ring takes whole subjects also where their items are
+             * tiles: with a tile's 2 chunks at a time half its waves idle (12
+             * subjects of 96..6000 trials, 5 % migration, tiles of 256: 446 us an
+             * iteration, with 64 chunks 265, whole subjects 252) */
+            const int64_t chunks = (ntr + kChunk - 1) / kChunk;
+            const int64_t ring = d.sub_mig > 0.0 ? std::min(64, std::max(1, 1024 / l.kchain)) : 1;
+            const int64_t tile = std::max<int64_t>(c.tpt / kChunk, ring);
+            max_chunks_item = std::max(max_chunks_item, nt == 1 ? chunks : std::min(chunks, tile));
         }
         l.rmax = std::max(l.rmax, nch);
         require(!c.span || span_fits(nch), "too many chain ranges per subject for items spanning every group");

@@ -109,3 +109,23 @@ def test_the_eight_wave_build_in_a_hierarchical_run(gpu):
         _same(want, got)
         assert np.array_equal(want[0]["phi"].theta, got[0]["phi"].theta)
         assert np.array_equal(want[0]["phi"].log_likelihoods, got[0]["phi"].log_likelihoods)
+
+
+@pytest.mark.parametrize("precision", ["MIXED_BATCHED", "FP64_BATCHED"])
+def test_migration_rings_of_tiled_subjects(gpu, precision):
+    # 71 chunks: a ring's likelihood takes more chunks at once than a tile has,
+    # in two rounds
+    fix = fx.load("lba_data6")
+    cells = [np.resize(fix.sub_data.rt[a:b], 9000 * (b - a) // len(fix.sub_data.rt))
+             for a, b in zip(fix.sub_data.cell_off[:-1], fix.sub_data.cell_off[1:])]
+    data = gpu.SubjectData.from_cells(cells)
+    assert 64 * 128 < len(data.rt)
+    rng = np.random.default_rng(4)
+    th = fx.truth_vector(fix)[:, None] * np.exp(rng.normal(0, 0.02, (fix.P, 12)))
+    lp = np.array([priors.sumlogprior(fix.sub_prior, th[:, c]) for c in range(12)])
+    start = (th, lp, gpu.loglike(fix.model, data, th.T.copy(), gpu.FP64_PLAIN))
+    jobs = [gpu.JobSpec(gpu.KIND_SUBJECT, 11 + s, fix.sub_prior, subject=data, start=start) for s in range(2)]
+    cfg = dict(nmc=12, nchain=12, sub_migration_prob=0.4, precision=getattr(gpu, precision))
+    want = _session(gpu, dict(cfg, launch_mode=1, chains_per_item=2), fix.model, jobs)
+    for k, tpt, mode in ((1, 128, 1), (2, 256, 2), (0, 256, 2), (4, 1024, 2), (2, 256, 3)):
+        _same(want, _session(gpu, dict(cfg, launch_mode=mode, chains_per_item=k, trials_per_tile=tpt), fix.model, jobs))
