@@ -830,7 +830,12 @@ ggdmc_session::Layout ggdmc_session::layout(Decomp c) const {
     while (l.cmax > 1 && bytes() > soft) l.cmax = (l.cmax + 1) / 2;
     if (bytes() > soft) l.tstage = 0;
     l.sweep_lds = bytes();
-    require(l.sweep_lds <= limit, "design too large for LDS (chains x parameters)");
+    /* at the limit chain_batch is 1; the tenth word of its constants is not
+     * counted, so that designs which fit with nine are taken (256 pairs and 64
+     * parameters: 44 chains, with the tenth 40). 66 KB, and the tables' 2, are
+     * well below what a workgroup may have, and two workgroups fit a CU. */
+    const size_t spare = sizeof(double) * (size_t)per_chain;
+    require(l.sweep_lds <= limit + spare, "design too large for LDS (chains x parameters)");
     /* the population step of each chain group runs in that group's subject
      * launch (not with one item per subject over every group, nor with
      * blocked subject sweeps: those keep the population kernel) */
@@ -843,9 +848,10 @@ ggdmc_session::Layout ggdmc_session::layout(Decomp c) const {
         bool whole_run = d.blocked_pop != 0 || d.pop_mig > 0.0;
         for (const ggdmc_job &j : jobs) whole_run = whole_run || j.kind == GGDMC_KIND_HYPER;
         l.ovl_stats_lds = ggdmc_internal_phi_lds(n, d.P, G, 1) <= limit ? 1 : 0;
-        l.ovl_lds = std::max({l.sweep_lds, whole_run ? ggdmc_internal_phi_lds(n, d.P, G, l.ovl_stats_lds) : (size_t)0,
-                              ggdmc_internal_phi_chain_lds(d.P, max_sub)});
-        l.overlap = l.ovl_lds <= limit;
+        const size_t phi = std::max(whole_run ? ggdmc_internal_phi_lds(n, d.P, G, l.ovl_stats_lds) : (size_t)0,
+                                    ggdmc_internal_phi_chain_lds(d.P, max_sub));
+        l.ovl_lds = std::max(l.sweep_lds, phi);
+        l.overlap = phi <= limit;
     }
     require(c.ipl == 1 || d.n_phi == 0 || l.overlap,
             "several iterations per launch need the population step inside the subject launch");

@@ -129,3 +129,58 @@ def test_migration_rings_of_tiled_subjects(gpu, precision):
     want = _session(gpu, dict(cfg, launch_mode=1, chains_per_item=2), fix.model, jobs)
     for k, tpt, mode in ((1, 128, 1), (2, 256, 2), (0, 256, 2), (4, 1024, 2), (2, 256, 3)):
         _same(want, _session(gpu, dict(cfg, launch_mode=mode, chains_per_item=k, trials_per_tile=tpt), fix.model, jobs))
+
+
+def _wide_design(gpu, P, ntrial, seed):
+    """256 condition x accumulator pairs and P parameters: thresholds (and
+    onsets) by condition, 8 accumulators."""
+    nq, na = 32, 8
+    src = np.full((nq, na, na, 6), -1, np.int32)       # condition, response, accumulator, family
+    cst = np.zeros(src.shape)
+    q = np.arange(nq)[:, None, None]
+    nb = min(32, P - 4)                                # thresholds; the rest are onsets
+    src[..., 0] = 0
+    src[..., 1] = 1 + q % nb
+    match = (np.arange(nq) % na)[:, None, None] == np.arange(na)[None, None, :]
+    src[..., 2] = np.where(match, 1 + nb, 2 + nb)
+    cst[..., 3] = 1.0
+    src[..., 5] = 3 + nb + q % (P - 3 - nb)
+    # (conditions that share every parameter would merge: sd_v tells them apart)
+    cst[..., 3] += 1e-3 * q
+    m = gpu.LBAModel(np.tile(np.arange(na), nq).astype(np.int32), src.reshape(nq * na, na, 6),
+                     cst.reshape(nq * na, na, 6), ["p%d" % i for i in range(P)])
+    x = np.full(P, 1.2)
+    x[0], x[1 + nb], x[2 + nb] = 0.4, 3.0, 1.0
+    x[3 + nb:] = 0.1
+    rng = np.random.default_rng(seed)
+    data = gpu.SubjectData.from_cells([rng.uniform(0.4, 1.5, ntrial) for _ in range(nq * na)])
+    return m, x, data
+
+
+@pytest.mark.parametrize("P,nchain", [(64, 44), (40, 75), (20, 150)])
+def test_the_largest_designs_that_lds_holds(gpu, P, nchain):
+    m, x, data = _wide_design(gpu, P, 1, P)
+    rng = np.random.default_rng(1)
+    prior = gpu.PriorSpec.uniform(P, 0.0, 10.0)
+
+    def job(n):
+        th = x[:, None] * np.exp(rng.normal(0, 0.02, (P, n)))
+        lp = np.array([priors.sumlogprior(prior, th[:, c]) for c in range(n)])
+        return gpu.JobSpec(gpu.KIND_SUBJECT, 7, prior, subject=data,
+                           start=(th, lp, gpu.loglike(m, data, th.T.copy(), gpu.FP64_PLAIN)))
+
+    most = job(nchain)
+    # (the stored likelihoods are the ones that loglike gives, bit for bit)
+    for prec, ll_prec in ((gpu.MIXED_BATCHED, gpu.MIXED_BATCHED), (gpu.FP64_BATCHED, gpu.FP64_PLAIN)):
+        cfg = dict(nmc=40, nchain=nchain, precision=prec)
+        got = gpu.run_batch(gpu.make_config(**cfg), m, [most])
+        _same(got, _session(gpu, dict(cfg, chains_per_item=1, launch_mode=3), m, [most]))
+        p = got[0]["subjects"][0]
+        moved = np.any(p.theta[:, :, -1] != p.theta[:, :, 0], axis=0)
+        assert moved.any()
+        ll = gpu.loglike(m, data, p.theta[:, moved, -1].T.copy(), ll_prec)
+        assert np.array_equal(ll, p.log_likelihoods[moved, -1])
+    plain = gpu.run_batch(gpu.make_config(3, nchain, precision=gpu.FP64_PLAIN), m, [most])[0]["subjects"][0]
+    assert np.isfinite(plain.log_likelihoods).all()
+    with pytest.raises(gpu.GgdmcError, match="too large for LDS"):
+        gpu.run_batch(gpu.make_config(3, nchain + 1), m, [job(nchain + 1)])
