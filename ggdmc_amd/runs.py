@@ -263,6 +263,7 @@ class _Batch:
                 cj.hyper_data = ptr(hd)
             else:
                 S = len(subjects)
+                starts = list(starts)
                 if len(starts) != S:
                     raise ValueError("%d start states for %d subjects" % (len(starts), S))
                 cj.nsubject = S
