@@ -1073,11 +1073,15 @@ bool ggdmc_session::try_decomp(const Decomp &c) {
  *   1024 x 2048 of 4 accumulators (1024 with all): -, 1209, 1074, 1068, 999
  * So: all chains of a group when the subjects alone fill the chip; else the
  * smallest k that keeps 3 items a CU, while that is at most 4; else the smallest
- * k from 4 that keeps 6.25 a CU, with 4 waves. The first candidate is within 13 %
- * of the best of about 45 on 20 workloads, and one of the list is the best or
- * within 3 % of it: its neighbours in k, launch mode and build follow, and trial
- * tiles where few long subjects leave the chip idle (1 x 4096, 18 chains: tiles
- * of 256 41 us, whole subjects 50). */
+ * k from 4 that keeps 6.25 a CU, with 4 waves. Its neighbours in k, launch mode
+ * and build follow, and trial tiles, first in the list, where few long subjects
+ * leave the chip idle (1 x 40000, 39 chains: tiles of 256 199 us, whole subjects
+ * with 8 waves 226, with 4 319). The list has at most eleven. Its first, which
+ * runs of fewer than six launches take, was within 9 % of its best on 20 of 27
+ * workloads (those above, 1 to 32 subjects of 64 to 40000 trials, FP64, 3 and 39
+ * groups, blocked, migration); not on 3 x 20000 (13 %), 1 x 4096 (tiles 43 us, 8 waves 36),
+ * 2000 x 100 (117, 98), 6 x 2500 (49, 41), 12 x 96..6000 (88, 67), 1 x 2100 (37,
+ * 27), 700 x 100 (57, 39). */
 std::vector<ggdmc_session::Decomp> ggdmc_session::candidates() const {
     const int ng = (d.nchain + d.G - 1) / d.G;
     const int64_t cus = std::max(device_cus(), 1);

@@ -84,11 +84,9 @@ namespace ggdmc {
 
 constexpr double kFloor = 1e-10;
 constexpr double kLogFloor = -23.025850929940457;          /* log(1e-10)           */
-constexpr double kLogDblEps = -36.04365338911715;          /* log(2.220446e-16)   */
 constexpr double kInvSqrt2Pi = 0.3989422804014327;
 constexpr double kLog2e = 1.4426950408889634;
 constexpr double kLn2 = 0.6931471805599453;
-constexpr double kSqrt1_2 = 0.7071067811865476;
 constexpr double kMillsK = 0.2625;
 constexpr int kMillsDeg = 10;
 /* R(z) ~= t * sum_{k=0}^{10} c_k t^k, t = 1/(1 + 0.2625 z), z >= 0 */
@@ -332,14 +330,14 @@ GGDMC_FN void naive_pdf_cdf(const AccK &k, double t, double &pdf, double &cdf) {
     cdf = naive_cdf<Ops>(k, t);
 }
 
-/* Error model of the mixed evaluation: every computed tail and exp(-z^2/2)
- * carries a relative error of up to kTailErr (FP32 exp2); a result whose
+/* Error model of the mixed evaluation: a computed tail carries a relative error
+ * of up to kTailErr, exp(-z^2/2) of up to kExpErr; a result whose
  * bound exceeds kCondTol relative, or whose reference FP64 value carries more
  * rounding noise than that where the rounding is not reproduced (Phi rounded
  * near 1, ulp 1.1e-16, scaled by the formula's coefficients), is flagged
  * ill-conditioned and the trial is evaluated with the reference's FP64
  * formula instead. */
-constexpr double kTailErr = 1e-9;   /* Mills-ratio fit (2.9e-10) and the FP32 seeds */
+constexpr double kTailErr = 1e-9;   /* the Mills-ratio fit (2.9e-10; measured with the rest under 4e-10) */
 constexpr double kExpErr = 1e-15;   /* exp(-z^2/2) in FP64 arithmetic */
 constexpr double kCondTol = 1e-5;
 constexpr double kUlp1 = 1.1102230246251565e-16;

@@ -96,12 +96,6 @@ enum { MODE_MIXED = 0, MODE_NAIVE = 1 };
 constexpr int kAccKDoubles = sizeof(AccK) / sizeof(double);
 
 /* --------------------------------------------------------------- likelihood */
-template <int MODE>
-__device__ __forceinline__ double trial_term(const AccK *kc, int n_acc, int w, double rt) {
-    return MODE == MODE_MIXED ? mixed_trial_term<DevOps>(kc, n_acc, w, rt)
-                              : naive_trial_term<DevOps>(kc, n_acc, w, rt);
-}
-
 /* x of another lane of the wave: a DPP move within a row of 16 lanes, or the
  * other half / neighbouring row by the gfx950 lane swaps (the two results of a
  * swap of x with itself hold, per lane, x of the lane's own and of its partner
@@ -1767,12 +1761,14 @@ __device__ __forceinline__ void late_prior(const Dev &d, const JobDev &job, cons
 /* ------------------------------------------------------------ sweep kernel */
 /* BLOCK: 512 (8 waves, at most one workgroup a CU) where the items are few and
  * hold more chunks than 4 waves take at once. OCC: waves per SIMD the kernel is
- * built for (3: up to 168 VGPRs a lane, 4:
- * 128, with values of the cold paths in scratch). LEAN: for launches whose every
+ * built for (2 with 512 threads; 3: up to 168 VGPRs a lane; 4: 128, with values
+ * in scratch: 36 VGPRs spilled in the LEAN build of the batched arithmetic, 73 in
+ * the general one, on the subjects' path as well: their slots are most of the
+ * HBM writes of the ragged workload below). LEAN: for launches whose every
  * iteration is a plain crossover of whole subjects (no migration, blocked
  * sweep, hyper-only run, trial tile or decision trace): without the migration
- * ring's and the whole-run population step's copies of the code the kernel is 87
- * KB instead of 230 and its path fits the 64 KB instruction cache of a CU pair
+ * ring's and the whole-run population step's copies of the code the kernel is 84
+ * KB instead of 200 and its path fits the 64 KB instruction cache of a CU pair
  * more often, which bounds an iteration of few subjects as much as its
  * arithmetic (us an iteration, general and lean: 18-chain fit 22.7 and 20.5,
  * 32 x 768 32.9 and 29.8, FP64 41.0 and 37.7, 256 ragged + 64 fits 144 and
@@ -2128,7 +2124,7 @@ __global__ __launch_bounds__(kBlock) void plain_subject_kernel(Dev d, uint32_t i
     double acc = 0.0;
     for (int64_t i = t_lo + threadIdx.x; i < t_hi; i += blockDim.x) {
         const int code = d.tcode[i];
-        acc += trial_term<MODE_NAIVE>(acck + (code >> 3) * d.n_acc, d.n_acc, code & 7, d.rt[i]);
+        acc += naive_trial_term<DevOps>(acck + (code >> 3) * d.n_acc, d.n_acc, code & 7, d.rt[i]);
     }
     const double tll = block_sum(acc, red);
     if (threadIdx.x == 0) {
