@@ -29,7 +29,8 @@ def test_every_split_gives_the_same_bits(gpu, ntrial, precision):
     data = _data(gpu, fix, ntrial)
     base = fx.near_thetas(fix, 7, seed=ntrial)
     one = np.array([gpu.loglike(fix.model, data, x[None], prec)[0] for x in base])
-    # 3, 31 and 300 vectors take other splits than one; 2700 share workgroups
+    # 300 vectors take another split than one (3 and 31 of up to 5000 trials the
+    # same: 8 chunks a workgroup; 31 of 35000 another); 2700 share workgroups
     for n in (3, 31, 300, 2700) if ntrial <= 1025 else (3, 31, 300):
         idx = np.arange(n) % 7
         got = gpu.loglike(fix.model, data, base[idx], prec)
@@ -46,3 +47,18 @@ def test_fixed_staging_takes_what_it_took_before_the_split(gpu):
     th = fx.near_thetas(fix, 40, seed=1)
     got = gpu.loglike(fix.model, data, th, gpu.MIXED_BATCHED, noalloc=True)
     assert np.array_equal(got, gpu.loglike(fix.model, data, th, gpu.MIXED_BATCHED))
+
+
+@pytest.mark.parametrize("precision", ["MIXED_BATCHED", "FP64_PLAIN"])
+@pytest.mark.parametrize("n,ntrial", [(200, 1100), (200, 1634), (400, 640), (400, 1250), (300, 1793), (500, 2146)])
+def test_uneven_splits_give_the_same_bits(gpu, n, ntrial, precision):
+    # 9, 13, 10, 15 and 17 chunks over 3, 4, 2, 4 and 2 workgroups, the last of
+    # most short of the others; 5 chunks in one
+    prec = getattr(gpu, precision)
+    fix = fx.load("lba_data6")
+    data = _data(gpu, fix, ntrial)
+    base = fx.near_thetas(fix, 5, seed=ntrial)
+    one = np.array([gpu.loglike(fix.model, data, x[None], prec)[0] for x in base])
+    idx = np.arange(n) % 5
+    assert np.array_equal(gpu.loglike(fix.model, data, base[idx], prec), one[idx])
+    assert np.array_equal(gpu.loglike(fix.model, data, base[idx], prec, noalloc=True), one[idx])
