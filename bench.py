@@ -52,21 +52,21 @@ W_ALG = {2: 130.0, 4: 255.0}
 # SIMD of the kernel build), for the
 # decompositions the autotuner picks on these workloads: a figure is reported
 # only for the decomposition it was counted on.
-W_ISSUED = {('c3', 1, 0, 4, 3): 477.4,
-            ('c3', 1, 0, 3, 3): 547.4,
-            ('c4', 4, 0, 4, 4): 333.0,
-            ('c4', 4, 0, 3, 4): 346.8,
-            ('c5', 17, 0, 4, 3): 497.6,
-            ('c5', 17, 0, 3, 3): 499.0}
+W_ISSUED = {('c3', 1, 0, 4, 3): 467.6,
+            ('c3', 1, 0, 3, 3): 535.8,
+            ('c4', 4, 0, 4, 4): 331.3,
+            ('c4', 4, 0, 3, 4): 343.5,
+            ('c5', 17, 0, 4, 3): 496.1,
+            ('c5', 17, 0, 3, 3): 497.1}
 # HBM bytes per iteration of the subject sweep kernel at those decompositions:
 # rocprofv3 FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 KiB (factors of a 256 MiB copy
 # kernel, same files) per launch, divided by the 32 iterations of a launch.
-TRAFFIC = {('c3', 1, 0, 4, 3): 1.390e+06,
-           ('c3', 1, 0, 3, 3): 1.200e+06,
-           ('c4', 4, 0, 4, 4): 2.536e+07,
-           ('c4', 4, 0, 3, 4): 4.205e+07,
-           ('c5', 17, 0, 4, 3): 2.121e+07,
-           ('c5', 17, 0, 3, 3): 2.029e+07}
+TRAFFIC = {('c3', 1, 0, 4, 3): 1.365e+06,
+           ('c3', 1, 0, 3, 3): 1.194e+06,
+           ('c4', 4, 0, 4, 4): 2.556e+07,
+           ('c4', 4, 0, 3, 4): 4.166e+07,
+           ('c5', 17, 0, 4, 3): 2.084e+07,
+           ('c5', 17, 0, 3, 3): 2.002e+07}
 # Iterations a bench session holds at least, whatever --steps asks: the
 # library autotunes the work decomposition of sessions of 64 or more
 # iterations, so the measured configuration never depends on the step count.

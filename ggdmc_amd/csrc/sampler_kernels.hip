@@ -1400,7 +1400,7 @@ __global__ __launch_bounds__(kPhiBlock) void phi_kernel(Dev d, uint32_t iter_off
  * its subjects are fixed data, so nothing outside the workgroup is read between
  * iterations and the state stays in LDS for the launch. One launch an iteration
  * staged and wrote it back each time: 14.7 us an iteration with 39 chains and 26
- * parameters, 9.4 here, bound by the chain of barriers, logarithms and draws of
+ * parameters, 8.7 here, bound by the chain of barriers, logarithms and draws of
  * two dependent chain groups in one workgroup. */
 __global__ __launch_bounds__(kPhiBlock) void hyper_kernel(Dev d, uint32_t iter0, int count, int stats_lds) {
     extern __shared__ __attribute__((aligned(16))) char lds_raw[];
