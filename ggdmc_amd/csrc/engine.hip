@@ -174,7 +174,8 @@ int device_cus() {
  * subject with higher workgroup ids as well as lower ones. The items of a
  * subject lie within kXcd * ranges consecutive workgroups (XCD-aware order);
  * while that window fits one workgroup per CU every item it waits on is
- * resident or done, whatever else occupies the chip. */
+ * resident or done, alone or beside launches that do not wait for slots
+ * themselves (several that do: span_beside_others). */
 constexpr int kXcd = 8;
 bool span_fits(int ranges) { return kXcd * ranges <= device_cus(); }
 
@@ -1135,7 +1136,8 @@ std::vector<ggdmc_session::Decomp> ggdmc_session::candidates() const {
             add({false, std::min(2, ng), 256, true, 1, false, 3, false});
             add({false, 1, 256, true, 1, false, 3, false});
         }
-        if (few(k)) multi(k, span, 3, true);
+        /* one workgroup of 8 waves is resident on a CU */
+        if (few(k)) multi(k, span && span_beside_others(pw, d.S, (ng + k - 1) / k, cus), 3, true);
         multi(k, span, occ);
         if (d.G > 2) add({true, 0, 0, false, 1, false, 3, false});
         multi(k, !span, occ);

@@ -31,6 +31,18 @@ inline bool waits_fit(int64_t ntrial, int n_acc, bool fp64, int G, int k, int ri
     return iteration_us(ntrial, n_acc, fp64, G, k, ring_chains) < kMaxIterationUs;
 }
 
+/* Items that span every chain group wait for items of their subject with higher
+ * workgroup ids too. Those lie within min(8, subjects) x ranges consecutive
+ * ids, behind phi_wgs population workgroups; launches of other threads'
+ * sessions may hold every other slot while they wait for the same reason. As
+ * many launches as a process has hardware queues (4) cannot stop each other
+ * while each of them may hold a subject's items: then one of them has all of a
+ * subject's. Mode 3, whose items wait for lower ids only, needs no such bound
+ * (8 waves, 4 x 768: 23.2 us an iteration, mode 4 22.3). */
+inline bool span_beside_others(int64_t phi_wgs, int64_t subjects, int64_t ranges, int64_t slots) {
+    return 4 * (phi_wgs + std::min<int64_t>(8, subjects) * ranges) <= slots;
+}
+
 /* The split of a likelihood call of n vectors over nj chunks on `cus` CUs: k
  * vectors and jper chunks per workgroup of `threads`, its trials staged in LDS
  * or not. Per workgroup the constants take about 4 us whatever k, a chunk of

@@ -40,6 +40,10 @@ int host_waits_fit(int64_t ntrial, int n_acc, int fp64, int G, int k, int ring_c
     return ggdmc::waits_fit(ntrial, n_acc, fp64 != 0, G, k, ring_chains);
 }
 
+int host_span_beside_others(int64_t phi_wgs, int64_t subjects, int64_t ranges, int64_t slots) {
+    return ggdmc::span_beside_others(phi_wgs, subjects, ranges, slots);
+}
+
 // The split of a likelihood call: out = {vectors, threads, chunks per workgroup, staged}.
 void host_loglike_shape(int64_t n, int nj, int64_t cus, int may_split, int *out) {
     const ggdmc::LoglikeShape s = ggdmc::loglike_shape(n, nj, cus, may_split != 0);

@@ -1,5 +1,7 @@
 """Work decompositions at the edges of what fits: a candidate that does not fit
 is passed over, and no decomposition changes a bit."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -184,3 +186,31 @@ def test_the_largest_designs_that_lds_holds(gpu, P, nchain):
     assert np.isfinite(plain.log_likelihoods).all()
     with pytest.raises(gpu.GgdmcError, match="too large for LDS"):
         gpu.run_batch(gpu.make_config(3, nchain + 1), m, [job(nchain + 1)])
+
+
+def test_sessions_of_several_threads_run_beside_each_other(gpu):
+    # four small hierarchical runs at once take the 8-wave build, one workgroup a
+    # CU: together more workgroups than the chip holds
+    w = workloads.make("c3", scale=0.1)
+    assert len(w.jobs[0].subjects) == 3
+    jobs = [gpu.JobSpec(j.kind, j.seed + r, j.p_prior, h_prior=j.h_prior, phi_start=j.phi_start, subjects=j.subjects,
+                        subject_starts=j.subject_starts, nparameter_de=j.nparameter_de)
+            for j in w.jobs for r in range(4)]
+    cfg = gpu.make_config(500, w.nchain)
+    alone = [gpu.run_batch(cfg, w.model, [j]) for j in jobs]
+    got = [None] * 4
+
+    def run(r):
+        got[r] = gpu.run_batch(cfg, w.model, [jobs[r]])
+
+    ts = [threading.Thread(target=run, args=(r,)) for r in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for a, b in zip(alone, got):
+        _same(a, b)
+        assert np.array_equal(a[0]["phi"].theta, b[0]["phi"].theta)
+    s = gpu.Session(cfg, w.model, jobs[:1])
+    assert not (s.waves_per_simd() == 2 and s.decomposition()[3] == 4)
+    s.close()

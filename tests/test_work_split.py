@@ -39,6 +39,39 @@ def test_waits_are_bounded_by_one_iteration(case, fits):
     assert fits == (want < 50_000)
 
 
+def _stuck(phi_wgs, subjects, ranges, slots, launches=4):
+    """Whether `launches` equal launches, given slots in turn, come to hold them
+    all without one subject's items together: segment order is phi_wgs population
+    workgroups, then the items, subjects in turn by workgroup id mod 8."""
+    left = {x: ranges for x in range(subjects)}
+    order = [None] * phi_wgs
+    while any(left.values()):
+        want = len(order) % 8
+        x = next(b for d in range(8) for b in sorted(left) if b % 8 == (want + d) % 8 and left[b])
+        left[x] -= 1
+        order.append(x)
+    held = min(len(order), slots // launches)
+    seen = [order[:held].count(x) for x in range(subjects)]
+    return held < len(order) and max(seen) < ranges
+
+
+@pytest.mark.parametrize("phi_wgs,subjects,ranges", [(0, 1, 9), (0, 1, 20), (0, 1, 128), (0, 3, 20), (0, 8, 16),
+                                                     (18, 1, 9), (18, 5, 9), (39, 1, 20), (39, 2, 20), (39, 3, 20),
+                                                     (39, 4, 20), (33, 5, 17), (7, 12, 4), (48, 1, 24)])
+def test_spanning_items_of_several_launches_cannot_stop_each_other(phi_wgs, subjects, ranges):
+    L = _lib()
+    L.host_span_beside_others.argtypes = [C.c_int64] * 4
+    ok = bool(L.host_span_beside_others(phi_wgs, subjects, ranges, 256))
+    assert ok == (4 * (phi_wgs + min(8, subjects) * ranges) <= 256)
+    if ok:
+        assert not any(_stuck(phi_wgs, subjects, ranges, 256, n) for n in (1, 2, 3, 4))
+
+
+def test_four_small_hierarchical_launches_of_eight_waves_would():
+    # what the rule is there for: 3 subjects x 20 ranges, 39 population workgroups
+    assert _stuck(39, 3, 20, 256) and not _lib().host_span_beside_others(39, 3, 20, 256)
+
+
 def _shape(n, nj, cus=256, may_split=True):
     out = (C.c_int * 4)()
     L = _lib()
